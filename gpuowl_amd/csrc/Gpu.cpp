@@ -4,11 +4,14 @@
 #include "Trig.h"
 #include "TrigBufCache.h"
 #include "Tune.h"
+#include "coltab.h"
 
 #include <algorithm>
 #include <chrono>
 #include <cmath>
 #include <cstring>
+#include <map>
+#include <mutex>
 
 namespace {
 
@@ -16,6 +19,20 @@ u32 pow2AtLeast(u32 x, u32 lo, u32 hi) {
   u32 t = lo;
   while (t < x && t < hi) { t *= 2; }
   return t;
+}
+
+// Compute units of a device, asked for once.
+u32 computeUnits(int device) {
+  static std::mutex mtx;
+  static std::map<int, u32> known;
+  std::lock_guard<std::mutex> lock(mtx);
+  u32& n = known[device];
+  if (!n) {
+    int cus = 0;
+    owlCheck(owl_hip_device_info(device, nullptr, 0, nullptr, nullptr, &cus, nullptr), "device info");
+    n = u32(std::max(cus, 1));
+  }
+  return n;
 }
 
 }  // namespace
@@ -116,10 +133,10 @@ Gpu::Gpu(u32 E, const FFTConfig& fftIn, const GpuOptions& optIn) : E{E}, fft{fft
   rowKernel = "rowx" + std::to_string(W) + "r" + std::to_string(R);
   bool rowFixed = !opt.generic && haveKernel(rowKernel);
   rowChunked = rowFixed && nb >= 8;
-  // column pass: k_colx (both columns in LDS) unless the one-region k_coly is asked for
-  // or k_colx's lane mapping does not fit ((H/16) % R == 0); then k_coly if compiled
+  // column pass: k_colx (both columns at once) unless the one-region k_coly is asked for
+  // or k_colx's addressing does not fit (R divides the butterflies of its first stage); then k_coly if compiled
   const std::string colY = "coly" + std::to_string(H), colX = "colx" + std::to_string(H);
-  bool useX = !opt.generic && !opt.colOneRegion && haveKernel(colX) && (H / 16) % R == 0;
+  bool useX = !opt.generic && !opt.colOneRegion && haveKernel(colX) && (H / colRadices(H).c0) % R == 0;
   bool useY = !opt.generic && !useX && haveKernel(colY);
   colKernel = useY ? colY : colX;
   bool colFixed = useY || useX;
@@ -153,19 +170,15 @@ Gpu::Gpu(u32 E, const FFTConfig& fftIn, const GpuOptions& optIn) : E{E}, fft{fft
     owl_kernel k = nullptr;
     owlCheck(owl_hip_kernel_get(colKernel.c_str(), &k), "kernel");
     owlCheck(owl_hip_kernel_max_threads(k, &colT), "kernel");
-    // the column regions + a colTwSize<H>()-entry twiddle table (kfixed.h)
-    const u32 twSize = 68 + H / 64 + 2 * (64 + H / 64 + 16);
-    // the two-region pass adds exact root tables for H >= 2304 (colRootSlots<H>())
-    const u32 rootSlots = (!useY && H >= 2304) ? 16 * 15 + (H == 4096 ? 0 : 16 * ((H / 256 - 1) | 1) + 240 + H / 16) : 0;
-    // two colRegionX<H>() regions (k_colx) or one colRegion<H>() (k_coly)
-    colLds = ((useY ? H + H / 16 + 4 : 2 * (H + 4)) + twSize + rootSlots) * 16;
-    if (useX && !opt.colOnePair && haveKernel(colX + "m")) {
-      int cus = 0, lds = 0;
-      owlCheck(owl_hip_device_info(opt.device, nullptr, 0, nullptr, nullptr, &cus, &lds), "device info");
-      colMulti = true;
-      colLdsM = colLds + twSize * 16;  // the next pair's twiddle table
-      slotsM = u32(std::max(cus, 1)) * std::max<u32>(1, u32(lds) / colLdsM);
+    if (useX) {
+      colLds = colSlotsX(H, false) * 16;
+      colSplitLds = colSlotsX(H, true) * 16;
+      haveSplit = !opt.colOnePair && haveKernel(colX + "m");
+    } else {
+      // colRegion<H>() + a colTwSize<H>()-entry twiddle table (kfixed.h)
+      colLds = (H + H / 16 + 4 + 68 + H / 64 + 2 * (64 + H / 64 + 16)) * 16;
     }
+    colX_ = useX;
   } else {
     colKernel = "col" + std::to_string(colT);
   }
@@ -219,6 +232,8 @@ Gpu::Gpu(u32 E, const FFTConfig& fftIn, const GpuOptions& optIn) : E{E}, fft{fft
   J.twMidB = trig_->midB.get();
   J.twPair = trig_->pair.get();
   J.twMidS = trig_->midS.get();
+  J.twMidM = trig_->midM.get();
+  J.colTab = trig_->colTab.get();
   J.lineW = upload(lineW);
   J.colW = upload(colW);
   J.rowMeta = nullptr;
@@ -277,7 +292,16 @@ Gpu::Gpu(u32 E, const FFTConfig& fftIn, const GpuOptions& optIn) : E{E}, fft{fft
   kRow = Kernel(rowKernel);
   colOne_ = colKernel;
   kCol = Kernel(colOne_);
-  if (colMulti) { kColM = Kernel(colOne_ + "m"); }
+  if (colX_) {
+    const std::string h = std::to_string(H);
+    kColSq[0][0] = Kernel("colcp" + h);
+    kColSq[0][1] = Kernel("colcn" + h);
+    if (haveSplit) {
+      kColSq[1][0] = Kernel("colx" + h + "m");
+      kColSq[1][1] = Kernel("colsn" + h);
+    }
+  }
+  cus_ = computeUnits(opt.device);
   colKernel = colKernelFor(1);
   kCarryB = Kernel("carryB");
   kCarryFix = Kernel("carryFix");
@@ -407,31 +431,28 @@ void Gpu::carryAll(Buf b, Launch L) {
   kCarryFix(L.q, 1, L.n, 256, 0, {&L.jobs, &wi, &co});
 }
 
-// Pairs per column group for a launch of nJobs jobs: the largest power of two up to
-// kMaxPairs whose grid (W/2 / pairs groups per job) still gives each of the device's
-// slotsM group slots a group; 1 when the multi-pair pass is not available. (At 7.5M words
-// two pairs per group take the column pass from 60.2 to 55.3 us; in 64-job batches of
-// 1.5M words, 2, 4, 8 or 16 pairs were within 2% of one pair and not kept for H < 2304.)
-u32 Gpu::colPairsPerGroup(u32 nJobs) const {
-  constexpr u32 kMaxPairs = 2;
-  u32 best = 1;
-  if (!colMulti) { return best; }
-  for (u32 p = 2; p <= kMaxPairs && p <= W / 2; p *= 2) {
-    if (u64(W / 2 / p) * nJobs < slotsM) { break; }
-    best = p;
-  }
-  return best;
+// Whether a column launch of nJobs jobs streams the state with non-temporal accesses: when the states together fit the
+// L2s (which then write back early instead of at the end of the launch) and when they exceed the 256 MB
+// Infinity Cache. Between, and below 6 MB, plain accesses are faster. Measured, us per squaring,
+// non-temporal / plain: 2 MB 16.4 / 15.7, 9.4 MB 31.2 / 33.8, 25 MB 37.0 / 40.1, 42 MB 56.3 / 57.9, 50 MB 64.8 / 65.2,
+// 63 MB 77.0 / 74.2; batches of 200 MB 262 / 235, 604 MB 639 / 692.
+bool Gpu::streamed(u32 nJobs) const {
+  const u64 bytes = 8ull * N * nJobs;
+  return bytes >= (6u << 20) && (bytes <= (56u << 20) || bytes > (256u << 20));
 }
 
-std::string Gpu::colKernelFor(u32 nJobs) const { return colPairsPerGroup(nJobs) > 1 ? colOne_ + "m" : colOne_; }
+// Whether a squaring column launch of nJobs jobs exchanges real and imaginary parts one after the other (four
+// waves per SIMD), compiled from H = 2304 up, where a group with complex exchanges takes
+// more than half of a CU's LDS: when the pairs give every CU two groups. (us per launch, split / complex:
+// 1024 x 3840 38.4 / 47.4, 256 x 2304 19.1 / 18.7. Below 2304 the complex exchange is faster in batches too.)
+bool Gpu::colSplit(u32 nJobs) const { return haveSplit && u64(W / 2) * nJobs >= 2 * cus_; }
+
+std::string Gpu::colKernelFor(u32 nJobs) const { return colSplit(nJobs) ? colOne_ + "m" : colOne_; }
 
 void Gpu::colPass(int mode, int fi, int oi, Launch L) {
-  const u32 p = colPairsPerGroup(L.n);
-  if (p > 1) {
-    kColM(L.q, W / 2 / p, L.n, colT, colLdsM, {&L.jobs, &mode, &fi, &oi});
-  } else {
-    kCol(L.q, W / 2, L.n, colT, colLds, {&L.jobs, &mode, &fi, &oi});
-  }
+  const bool split = mode == COL_SQUARE && colSplit(L.n);
+  const Kernel& k = colX_ && mode == COL_SQUARE ? kColSq[split][streamed(L.n)] : kCol;
+  k(L.q, W / 2, L.n, colT, split ? colSplitLds : colLds, {&L.jobs, &mode, &fi, &oi});
 }
 
 void Gpu::colSquare(Launch L) { colPass(COL_SQUARE, 0, 0, L); }

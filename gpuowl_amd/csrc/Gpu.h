@@ -45,7 +45,7 @@ struct GpuOptions {
   bool longCarry = false;  // lead-out + lead-in around every iteration (the reference's -carry long)
   bool generic = false;    // runtime-plan kernels even where a shape-specialized pass exists
   bool colOneRegion = false;  // the one-region column pass (k_coly) where k_colx exists
-  bool colOnePair = false;    // k_colx with one column pair per group where two would be chosen
+  bool colOnePair = false;    // k_colx without split exchanges, one column pair on a CU at a time
   u32 width = 0;           // W of the W x H split of the FFT; 0 = the reference's (refactored when too tall)
   u32 lineBlock = 0;       // lines per row-pass block; 0 = automatic
   int device = 0;
@@ -83,14 +83,13 @@ public:
   int device = 0;  // the HIP device the engine's queue and buffers are on
   u32 N, ND, W, H, R, nb, rowT, colT, rowLds, colLds;
   std::string rowKernel, colKernel;  // colKernel: what a launch of this job alone runs
-  bool rowChunked = false;           // fused row launches in chunked per-XCD block order (k_rowx, nb >= 8)
-  // Column pass with several column pairs per group ("colx<H>m", compiled for every k_colx
-  // shape): colLdsM bytes of LDS (one more twiddle table), slotsM = groups the device holds
-  // at once. colPairsPerGroup(n) is 1 (the one-pair "colx<H>") unless a launch of n jobs
-  // still gives every slot a group with fewer groups per job.
-  bool colMulti = false;
-  u32 colLdsM = 0, slotsM = 0;
-  u32 colPairsPerGroup(u32 nJobs) const;
+  bool rowChunked = false;           // fused row launches in chunked per-XCD block order (nb >= 8)
+  // Variants of the squaring's column pass, chosen per launch by its number of jobs: exchanges of real and imaginary
+  // parts one after the other (split) or of complex elements, plain or non-temporal (streamed) accesses.
+  bool haveSplit = false;
+  u32 colSplitLds = 0;  // LDS bytes of the split variant
+  bool colSplit(u32 nJobs) const;
+  bool streamed(u32 nJobs) const;
   std::string colKernelFor(u32 nJobs) const;  // the column kernel a launch of nJobs jobs runs
   bool useLongCarry;
   std::vector<u32> rowPlan, colPlan;
@@ -231,8 +230,11 @@ private:
   u32 stairTag_ = 0, lastTag_ = 0, resLo_ = 1, resHi_ = 0;
   u32 faultAt_ = 0;
   bool tunedLineBlock_ = false;
-  std::string colOne_;  // the one-pair column kernel
-  Kernel kRow, kCol, kColM, kCarryB, kCarryFix, kWordsIn, kWordsOut, kResidue, kIsEqual, kSum64, kCopy;
+  std::string colOne_;  // the column kernel without its "m" (split) suffix
+  bool colX_ = false;   // the column pass is k_colx
+  u32 cus_ = 1;         // compute units
+  Kernel kColSq[2][2];  // [split][streamed]: squaring column pass (colX_)
+  Kernel kRow, kCol, kCarryB, kCarryFix, kWordsIn, kWordsOut, kResidue, kIsEqual, kSum64, kCopy;
 
   template<typename T> T* alloc(size_t n);
   template<typename T> T* upload(const std::vector<T>& v);

@@ -1,6 +1,7 @@
 #include "TrigBufCache.h"
 
 #include "Trig.h"
+#include "coltab.h"
 
 #include <map>
 #include <mutex>
@@ -8,6 +9,26 @@
 
 namespace {
 double2 d2(std::pair<double, double> p) { return double2{p.first, p.second}; }
+
+// The entries of ColTab<H, C0, C1, C2> (coltab.h).
+std::vector<double2> colTabOf(u32 H) {
+  const ColRadices r = colRadices(H);
+  if (!r.c0) { return {}; }
+  const u32 KS = (r.c1 - 1) | 1, ROOTS = 256;
+  std::vector<double2> t(colTabLds(H) + 6 * ROOTS, double2{0, 0});
+  auto product = [&](u32 at, u32 rows, u32 n) {  // w_n^(p*k), p < rows, 1 <= k < C1
+    for (u32 p = 0; p < rows; ++p) {
+      for (u32 k = 1; k < u32(r.c1); ++k) { t[at + p * KS + k - 1] = d2(root1(n, p * k)); }
+    }
+  };
+  product(0, r.c0, r.c0 * r.c1);
+  if (r.c2 != r.c0) { product(r.c0 * KS, r.c2, r.c2 * r.c1); }
+  const u32 m[6] = {1, 2, 3, 4, 8, 12};
+  for (u32 i = 0; i < 6; ++i) {
+    for (u32 k = 0; k < ROOTS; ++k) { t[colTabLds(H) + i * ROOTS + k] = d2(root1(H, m[i] * k)); }
+  }
+  return t;
+}
 }  // namespace
 
 std::shared_ptr<const TrigTables> TrigBufCache::get(u32 W, u32 H, owl_queue q) {
@@ -36,6 +57,14 @@ std::shared_ptr<const TrigTables> TrigBufCache::get(u32 W, u32 H, owl_queue q) {
   t->midB = Buffer<double2>(q, midB);
   t->pair = Buffer<double2>(q, pair);
   t->midS = Buffer<double2>(q, midS);
+  if (const u32 c0 = colRadices(H).c0) {
+    std::vector<double2> midM(size_t(W) * 16);
+    for (u32 a = 0; a < W; ++a) {
+      for (u32 k = 0; k < 16; ++k) { midM[size_t(a) * 16 + k] = d2(root1(ND, u64(a) * k * (H / c0) % ND)); }
+    }
+    t->midM = Buffer<double2>(q, midM);
+    t->colTab = Buffer<double2>(q, colTabOf(H));
+  }
   cache[key] = t;
   return t;
 }

@@ -18,6 +18,8 @@ struct TrigTables {
   Buffer<double2> midB;   // W*ceil(H/64): exp(-2 pi i a*64*hi / ND)
   Buffer<double2> pair;   // W: exp(-2 pi i a / ND)
   Buffer<double2> midS;   // W*16: exp(-2 pi i a*k*(H/16) / ND)
+  Buffer<double2> midM;   // W*16: exp(-2 pi i a*k*(H/C0) / ND), C0 the mirrored column pass's first radix
+  Buffer<double2> colTab; // the mirrored column pass's table (coltab.h), empty where H has no such pass
 };
 
 class TrigBufCache {

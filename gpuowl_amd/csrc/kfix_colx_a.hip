@@ -1,17 +1,26 @@
-// Two-region column passes compiled per H (H < 2048): k_colx<H, T, 16, C1, C2> (forward plan
-// [16, C1, C2]). The host picks "colx<H>" when it exists and (H/16) % R == 0.
+// Column passes compiled per H (H < 2048): k_colx<H, T, C0, C1, C2, SPLIT, NT, SQ> with the radices and threads of
+// coltab.h. "colx<H>" runs every mode; the squaring alone: "colcp<H>" (complex exchanges, plain accesses),
+// "colcn<H>" (complex, non-temporal), and from H = 2304 up "colx<H>m" (split exchanges, plain) and "colsn<H>" (split,
+// non-temporal). Gpu::colPass chooses.
 #include "kfixed.h"
 
+#define PASS(NAME, H, SPLIT, NT, SQ) \
+  {NAME, (const void*)&k_colx<H, colThreadsX(H), colRadices(H).c0, colRadices(H).c1, colRadices(H).c2, SPLIT, NT, SQ>, \
+   colThreadsX(H)}
+#define COMPLEX(H) \
+  PASS("colx" #H, H, false, false, false), PASS("colcp" #H, H, false, false, true), PASS("colcn" #H, H, false, true, true)
+#define SPLIT(H) PASS("colx" #H "m", H, true, false, true), PASS("colsn" #H, H, true, true, true)
+
 extern "C" const OwlKernelEntry owl_kernel_table_colx_a[] = {
-    {"colx512", (const void*)&k_colx<512, 64, 16, 16, 2>, 64},
-    {"colx768", (const void*)&k_colx<768, 128, 16, 16, 3>, 128},
-    {"colx1024", (const void*)&k_colx<1024, 128, 16, 16, 4>, 128},
-    {"colx1152", (const void*)&k_colx<1152, 256, 16, 8, 9>, 256},
-    {"colx1280", (const void*)&k_colx<1280, 256, 16, 16, 5>, 256},
-    {"colx1408", (const void*)&k_colx<1408, 256, 16, 8, 11>, 256},
-    {"colx1536", (const void*)&k_colx<1536, 256, 16, 16, 6>, 256},
-    {"colx1664", (const void*)&k_colx<1664, 256, 16, 8, 13>, 256},
-    {"colx1792", (const void*)&k_colx<1792, 256, 16, 16, 7>, 256},
-    {"colx1920", (const void*)&k_colx<1920, 256, 16, 8, 15>, 256},
+    COMPLEX(512),
+    COMPLEX(768),
+    COMPLEX(1024),
+    COMPLEX(1152),
+    COMPLEX(1280),
+    COMPLEX(1408),
+    COMPLEX(1536),
+    COMPLEX(1664),
+    COMPLEX(1792),
+    COMPLEX(1920),
     {nullptr, nullptr, 0},
 };

@@ -1,16 +1,23 @@
-// Two-region column passes compiled per H (H >= 2048): k_colx<H, T, 16, C1, C2> (forward plan
-// [16, C1, C2]). The host picks "colx<H>" when it exists and (H/16) % R == 0.
+// Column passes compiled per H (2048 <= H < 3072): k_colx<H, T, C0, C1, C2, SPLIT, NT, SQ> with the radices and threads of
+// coltab.h. "colx<H>" runs every mode; the squaring alone: "colcp<H>" (complex exchanges, plain accesses),
+// "colcn<H>" (complex, non-temporal), and from H = 2304 up "colx<H>m" (split exchanges, plain) and "colsn<H>" (split,
+// non-temporal). Gpu::colPass chooses.
 #include "kfixed.h"
 
+#define PASS(NAME, H, SPLIT, NT, SQ) \
+  {NAME, (const void*)&k_colx<H, colThreadsX(H), colRadices(H).c0, colRadices(H).c1, colRadices(H).c2, SPLIT, NT, SQ>, \
+   colThreadsX(H)}
+#define COMPLEX(H) \
+  PASS("colx" #H, H, false, false, false), PASS("colcp" #H, H, false, false, true), PASS("colcn" #H, H, false, true, true)
+#define SPLIT(H) PASS("colx" #H "m", H, true, false, true), PASS("colsn" #H, H, true, true, true)
+
 extern "C" const OwlKernelEntry owl_kernel_table_colx_b[] = {
-    {"colx2048", (const void*)&k_colx<2048, 256, 16, 16, 8>, 256},
-    {"colx2304", (const void*)&k_colx<2304, 512, 16, 16, 9>, 512},
-    {"colx2560", (const void*)&k_colx<2560, 512, 16, 16, 10>, 512},
-    {"colx2816", (const void*)&k_colx<2816, 512, 16, 16, 11>, 512},
-    {"colx3072", (const void*)&k_colx<3072, 512, 16, 16, 12>, 512},
-    {"colx3328", (const void*)&k_colx<3328, 512, 16, 16, 13>, 512},
-    {"colx3584", (const void*)&k_colx<3584, 512, 16, 16, 14>, 512},
-    {"colx3840", (const void*)&k_colx<3840, 512, 16, 16, 15>, 512},
-    {"colx4096", (const void*)&k_colx<4096, 512, 16, 16, 16>, 512},
+    COMPLEX(2048),
+    COMPLEX(2304),
+    SPLIT(2304),
+    COMPLEX(2560),
+    SPLIT(2560),
+    COMPLEX(2816),
+    SPLIT(2816),
     {nullptr, nullptr, 0},
 };

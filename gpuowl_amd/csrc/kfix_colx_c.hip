@@ -1,17 +1,26 @@
-// Two-region column passes with several column pairs per group (k_colx<H, T, 16, C1, C2, true>),
-// compiled for the H whose k_colx needs more than half of a CU's LDS (H >= 2304), so that one
-// group runs per CU. The host runs "colx<H>m" in place of "colx<H>" when a launch has enough
-// groups to give every CU one with fewer groups per job (see Gpu::colPairsPerGroup).
+// Column passes compiled per H (H >= 3072): k_colx<H, T, C0, C1, C2, SPLIT, NT, SQ> with the radices and threads of
+// coltab.h. "colx<H>" runs every mode; the squaring alone: "colcp<H>" (complex exchanges, plain accesses),
+// "colcn<H>" (complex, non-temporal), and from H = 2304 up "colx<H>m" (split exchanges, plain) and "colsn<H>" (split,
+// non-temporal). Gpu::colPass chooses.
 #include "kfixed.h"
 
+#define PASS(NAME, H, SPLIT, NT, SQ) \
+  {NAME, (const void*)&k_colx<H, colThreadsX(H), colRadices(H).c0, colRadices(H).c1, colRadices(H).c2, SPLIT, NT, SQ>, \
+   colThreadsX(H)}
+#define COMPLEX(H) \
+  PASS("colx" #H, H, false, false, false), PASS("colcp" #H, H, false, false, true), PASS("colcn" #H, H, false, true, true)
+#define SPLIT(H) PASS("colx" #H "m", H, true, false, true), PASS("colsn" #H, H, true, true, true)
+
 extern "C" const OwlKernelEntry owl_kernel_table_colx_c[] = {
-    {"colx2304m", (const void*)&k_colx<2304, 512, 16, 16, 9, true>, 512},
-    {"colx2560m", (const void*)&k_colx<2560, 512, 16, 16, 10, true>, 512},
-    {"colx2816m", (const void*)&k_colx<2816, 512, 16, 16, 11, true>, 512},
-    {"colx3072m", (const void*)&k_colx<3072, 512, 16, 16, 12, true>, 512},
-    {"colx3328m", (const void*)&k_colx<3328, 512, 16, 16, 13, true>, 512},
-    {"colx3584m", (const void*)&k_colx<3584, 512, 16, 16, 14, true>, 512},
-    {"colx3840m", (const void*)&k_colx<3840, 512, 16, 16, 15, true>, 512},
-    {"colx4096m", (const void*)&k_colx<4096, 512, 16, 16, 16, true>, 512},
+    COMPLEX(3072),
+    SPLIT(3072),
+    COMPLEX(3328),
+    SPLIT(3328),
+    COMPLEX(3584),
+    SPLIT(3584),
+    COMPLEX(3840),
+    SPLIT(3840),
+    COMPLEX(4096),
+    SPLIT(4096),
     {nullptr, nullptr, 0},
 };

@@ -4,9 +4,8 @@
 // Same algorithm, layout and modes as k_row / k_col in kernels.hip, with the
 // FFT plan fixed at compile time (no integer division, no radix dispatch, every
 // loop unrolled) and fewer LDS round trips:
-//   k_colx: the first forward stage is fused with the global load and the mid
-//           twiddle, the last inverse stage with the conjugate twiddle and the
-//           store (forward plan [C0,C1,C2], inverse plan [C1,C2,C0]).
+//   k_colx: a butterfly of each of the pair's columns in registers from the load to the
+//           store, four LDS exchanges (forward plan [C0,C1,C2], inverse [C2,C1,C0]).
 //   k_rowx: the last inverse stage leaves each thread holding whole columns
 //           (T = W/F0 threads, columns tid + k*T for all R lines), so rounding,
 //           the carry chain, the stairway hand-off and the weighting all run in
@@ -20,32 +19,21 @@
 // FFT stages spread over the banks, and consecutive line (row pass) or column (column pass)
 // regions start 6 (row pass, 4 or 8 lines) or 4 elements apart mod 16, which keeps the writes
 // that span several regions (the row pass's slot-order scatter, the column pass's first stage)
-// on distinct slots mod 8.
+// on distinct slots mod 8. (8-byte accesses: a write serves 16 lanes per cycle, slots mod 16, a read 32
+// lanes, slots mod 32.)
 #pragma once
 
 #include <type_traits>
 
 #include "kcommon.h"
+#include "coltab.h"
+
+#define CONSTANT __attribute__((address_space(4)))
 
 __device__ __forceinline__ int padi(int i) { return i + (i >> 4); }
-// Column-pass region layout: element i at lx(i), the low three bits of i XORed with bits 4..6
-// (each 16-element run keeps its place, permuted), no padding. Consecutive elements read by a
-// half-wave stay in distinct bank quads within each read sub-group, and the R consecutive outputs
-// of a radix-R butterfly for 8 consecutive lanes (stride R across the lanes) land on 8 distinct
-// slots mod 8. (In the row pass, whose LDS phases overlap the other group's work, the padded layout
-// measured as fast: there the fewer address operations weigh as much as the fewer bank conflicts.)
-__device__ __forceinline__ int lx(int i) { return i ^ ((i >> 4) & 7); }
-template<bool XL> __device__ __forceinline__ int lpos(int i) {
-  if constexpr (XL) {
-    return lx(i);
-  } else {
-    return padi(i);
-  }
-}
 // region strides in 16-byte elements (the host sizes LDS with the same formulas)
 template<int W, int R> constexpr int rowRegion() { return W + W / 16 + ((R == 4 || R == 8) ? 6 : 4); }
-template<int H> constexpr int colRegion() { return H + H / 16 + 4; }  // k_coly (padded layout)
-template<int H> constexpr int colRegionX() { return H + 4; }          // k_colx (lx layout)
+template<int H> constexpr int colRegion() { return H + H / 16 + 4; }
 
 // One LDS -> LDS radix-R autosort stage over NFFT FFTs of length L stored in
 // padded regions; Ns is the product of the earlier radices. The twiddle of butterfly input k
@@ -58,7 +46,7 @@ template<int H> constexpr int colRegionX() { return H + 4; }          // k_colx 
 // reads across waves.
 template<int L, int T, int R, bool PRIV> constexpr bool stagePrivate() { return PRIV && (T == 64 || L / R == 64); }
 
-template<int L, int REG, int NFFT, int T, bool INV, int R, int Ns, bool PRIV = false, bool XL = false, class TW>
+template<int L, int REG, int NFFT, int T, bool INV, int R, int Ns, bool PRIV = false, class TW>
 __device__ __forceinline__ void xstage(T2* lds, const TW& tw, int tid) {
   constexpr bool priv = stagePrivate<L, T, R, PRIV>();
   constexpr int NB = L / R;
@@ -72,19 +60,7 @@ __device__ __forceinline__ void xstage(T2* lds, const TW& tw, int tid) {
     if (TOT % T == 0 || g < TOT) {
       const int f = g / NB, j = g % NB;
       const T2* x = lds + f * REG;
-      if constexpr (XL && NB % 128 == 0) {  // lx(j + k*NB) = lx(j) + k*NB
-        const T2* xj = x + lx(j);
-#pragma unroll
-        for (int k = 0; k < R; ++k) { v[m][k] = xj[k * NB]; }
-      } else if constexpr (XL && NB % 64 == 0) {  // lx(j + k*NB) = (lx(j) ^ 4*(k & 1)) + k*NB
-        const T2* x0 = x + lx(j);
-        const T2* x1 = x + (lx(j) ^ 4);
-#pragma unroll
-        for (int k = 0; k < R; ++k) { v[m][k] = (k & 1 ? x1 : x0)[k * NB]; }
-      } else if constexpr (XL) {
-#pragma unroll
-        for (int k = 0; k < R; ++k) { v[m][k] = x[lx(j + k * NB)]; }
-      } else if constexpr (NB % 16 == 0) {  // padi(j + k*NB) = padi(j) + k*(NB + NB/16)
+      if constexpr (NB % 16 == 0) {  // padi(j + k*NB) = padi(j) + k*(NB + NB/16)
         const T2* xj = x + padi(j);
 #pragma unroll
         for (int k = 0; k < R; ++k) { v[m][k] = xj[k * (NB + NB / 16)]; }
@@ -116,18 +92,7 @@ __device__ __forceinline__ void xstage(T2* lds, const TW& tw, int tid) {
       T2* x = lds + f * REG;
       const int p = j % Ns;
       const int base = (j - p) * R + p;
-      if constexpr (XL && Ns % 128 == 0) {  // lx(base + k*Ns) = lx(base) + k*Ns
-        T2* xb = x + lx(base);
-#pragma unroll
-        for (int k = 0; k < R; ++k) { xb[k * Ns] = v[m][k]; }
-      } else if constexpr (XL && Ns == 1 && 16 % R == 0) {  // base = j*R: lx(base + k) = lx(base) ^ k
-        const int lb = lx(base);
-#pragma unroll
-        for (int k = 0; k < R; ++k) { x[lb ^ k] = v[m][k]; }
-      } else if constexpr (XL) {
-#pragma unroll
-        for (int k = 0; k < R; ++k) { x[lx(base + k * Ns)] = v[m][k]; }
-      } else if constexpr (Ns % 16 == 0) {  // padi(base + k*Ns) = padi(base) + k*(Ns + Ns/16)
+      if constexpr (Ns % 16 == 0) {  // padi(base + k*Ns) = padi(base) + k*(Ns + Ns/16)
         T2* xb = x + padi(base);
 #pragma unroll
         for (int k = 0; k < R; ++k) { xb[k * (Ns + Ns / 16)] = v[m][k]; }
@@ -148,22 +113,21 @@ __device__ __forceinline__ void xstage(T2* lds, const TW& tw, int tid) {
   }
 }
 
-// XL: regions in the lx layout (row pass) instead of padi (column pass)
-template<int L, int REG, int NFFT, int T, bool INV, bool PRIV, bool XL, int Ns, int... Rs> struct XStages;
-template<int L, int REG, int NFFT, int T, bool INV, bool PRIV, bool XL, int Ns>
-struct XStages<L, REG, NFFT, T, INV, PRIV, XL, Ns> {
+template<int L, int REG, int NFFT, int T, bool INV, bool PRIV, int Ns, int... Rs> struct XStages;
+template<int L, int REG, int NFFT, int T, bool INV, bool PRIV, int Ns>
+struct XStages<L, REG, NFFT, T, INV, PRIV, Ns> {
   template<class TW> __device__ __forceinline__ static void run(T2*, const TW&, int) {}
 };
-template<int L, int REG, int NFFT, int T, bool INV, bool PRIV, bool XL, int Ns, int R, int... Rs>
-struct XStages<L, REG, NFFT, T, INV, PRIV, XL, Ns, R, Rs...> {
+template<int L, int REG, int NFFT, int T, bool INV, bool PRIV, int Ns, int R, int... Rs>
+struct XStages<L, REG, NFFT, T, INV, PRIV, Ns, R, Rs...> {
   template<class TW> __device__ __forceinline__ static void run(T2* lds, const TW& tw, int tid) {
-    xstage<L, REG, NFFT, T, INV, R, Ns, PRIV, XL>(lds, tw, tid);
+    xstage<L, REG, NFFT, T, INV, R, Ns, PRIV>(lds, tw, tid);
     if constexpr (sizeof...(Rs) > 0) {
       // a workgroup-wide stage after a wave-private one reads what other waves wrote
       constexpr int next[] = {Rs...};
       if constexpr (stagePrivate<L, T, R, PRIV>() && !stagePrivate<L, T, next[0], PRIV>()) { __syncthreads(); }
     }
-    XStages<L, REG, NFFT, T, INV, PRIV, XL, Ns * R, Rs...>::run(lds, tw, tid);
+    XStages<L, REG, NFFT, T, INV, PRIV, Ns * R, Rs...>::run(lds, tw, tid);
   }
 };
 
@@ -275,46 +239,13 @@ __device__ __forceinline__ void fillRowTw(const T2* twRow, T2* tab, int tid) {
 // footprint (and so the number of groups per CU) as low as the data allows.
 template<int H> constexpr int colTwPer() { return 64 + H / 64 + 16; }
 template<int H> constexpr int colTwSize() { return TA_SLOTS + H / 64 + 2 * colTwPer<H>(); }
-// With ROOTS (H >= 2304, plan [16, 16, H/256]), the second forward stage (Ns = 16, R = 16: 256th
-// roots) and the second inverse stage (Ns = 16, R = H/256: (H/16)-th roots) read exact product
-// tables (fillProd; roots, after the pair tables): A, 16 rows of stride 15, then B, 16 rows of stride
-// (H/256 - 1) | 1, unless H/16 = 256 and A serves both.
-// Below H = 4096 the stages whose twiddles are w_H^(p*k) (the last forward stage, Ns = 256, and the
-// last inverse stage, Ns = H/16) read them as P2[(p >> 4) * k] * P1[p & 15][k], as the row pass
-// does (P1: w_H^(t*k), 16 rows of stride 15; P2: w_H^(16 j), j < H/16), after B. (At H = 4096
-// they stay with TA and TB: the two-pair pass would not fit in LDS.)
-template<int H> constexpr int colProdStrideB() { return (H / 256 - 1) | 1; }
-template<int H> constexpr int colRootSlots() {
-  return 16 * 15 + (H == 4096 ? 0 : 16 * colProdStrideB<H>() + 240 + H / 16);
-}
-template<int H, bool ROOTS = false>
+template<int H>
 struct ColTw {
   static_assert(H % 64 == 0 && H / 64 <= 64, "twiddle table");
   static constexpr int MID = TA_SLOTS + H / 64;  // start of column 0's part
   const T2* tab;
-  const T2* roots = nullptr;
   __device__ __forceinline__ T2 operator()(int m) const { return cmul(tab[taPos(m & 63)], tab[TA_SLOTS + (m >> 6)]); }
-  static constexpr bool PK = ROOTS && H != 4096;
-  static constexpr int P1 = PK ? 16 * 15 + 16 * colProdStrideB<H>() : 0, P2 = P1 + 240;
-  // w_H^(p*k) for p*k < H and 1 <= k < 16
-  __device__ __forceinline__ T2 pk(int p, int k) const {
-    if constexpr (PK) {
-      return cmul(roots[P2 + (p >> 4) * k], roots[P1 + (p & 15) * 15 + k - 1]);
-    } else {
-      return (*this)(p * k);
-    }
-  }
-  template<int NR, int RR> __device__ __forceinline__ T2 st(int p, int k, int stride) const {
-    if constexpr (ROOTS && NR == 256 && RR == 16) {
-      return roots[p * 15 + k - 1];
-    } else if constexpr (ROOTS && NR == H / 16 && RR == H / 256) {
-      return roots[16 * 15 + p * colProdStrideB<H>() + k - 1];
-    } else if constexpr (NR == H && RR <= 16) {
-      return pk(p, k);
-    } else {
-      return (*this)(p * stride * k);
-    }
-  }
+  template<int NR, int RR> __device__ __forceinline__ T2 st(int p, int k, int stride) const { return (*this)(p * stride * k); }
   __device__ __forceinline__ T2 mid(int h, int l) const {
     const T2* p = tab + MID + h * colTwPer<H>();
     return cmul(p[l & 63], p[64 + (l >> 6)]);
@@ -348,217 +279,351 @@ template<int H>
 __device__ __forceinline__ void fillColTw(const JobDesc& J, T2* tab, int a0, int a1, int tid, int T) {
   for (int i = tid; i < colTwSize<H>(); i += T) { tab[i] = colTwEntry<H>(J, i, a0, a1); }
 }
-template<int H>
-__device__ __forceinline__ void fillColRoots(const JobDesc& J, T2* roots, int tid, int T) {
-  static_assert(H % 256 == 0 && H / 256 <= 16, "column product tables");
-  fillProd<16, 15, 15>(J.twCol, H / 256, roots, tid, T);
-  if constexpr (H != 4096) {
-    fillProd<16, H / 256 - 1, colProdStrideB<H>()>(J.twCol, 16, roots + 16 * 15, tid, T);
-    using TW = ColTw<H, true>;
-    fillProd<16, 15, 15>(J.twCol, 1, roots + TW::P1, tid, T);
-    for (int j = tid; j < H / 16; j += T) { roots[TW::P2 + j] = gld(J.twCol + 16 * j); }
+// ---------------------------------------------------------------- column pass, mirrored pair
+// The two columns of a pair have frequencies a and W - a. Transforming the conjugate of column
+// W - a takes exactly column a's twiddles (w_ND^(-(W-a)*l) = w_ND^(a*l) * w_H^(-l), and the w_H^(-l)
+// only shifts the output index), and its output b is conj(X_{W-a}[H-1-b]): the pairing partner
+// of X_a[b], already conjugated. So in a row of 16 lanes the first 8 run butterflies of column a and the
+// others the same butterflies of column W - a, with the same twiddles; after the last forward stage a
+// lane's partner bins are in the lane 8 away, and the pairing and the first inverse stage run in registers
+// (forward plan [C0, C1, C2], inverse [C2, C1, C0]; four LDS exchanges, where transforming both columns stage by
+// stage in LDS took six round trips).
+// One butterfly per thread. SPLIT: real and imaginary parts are exchanged one after the other through one region
+// of doubles per column, in at most 128 VGPRs, so that at H = 3840 two groups and four waves per SIMD share a CU;
+// otherwise whole complex elements, with half the barriers.
+// LDS positions are sums (one address per butterfly, the rest in the instructions' offsets) and free of
+// bank conflicts: rows of a Ns = 1 exchange are odd (C + 1 for even C), the blocks of the others C apart, so
+// that consecutive butterflies write distinct slots; the two columns' regions use different halves of the banks
+// and alternate by 16 lanes.
+// NT: non-temporal loads and stores.
+// Measured (HIP events, us per launch, the pass before it in parentheses): 1024 x 3840 split 38.4 (46.1), 1024 x 2560
+// split 29.4 (35.4), 1024 x 1536 19.1 (23.4), 256 x 2304 18.7 (20.3), 256 x 512 9.2 (13.5).
+// Values derived from i before and after are computed anew instead of being held in registers.
+#define FRESH(i) asm volatile("" : "+v"(i))
+// Fixes the place of the values in the instruction stream.
+template<int N> __device__ __forceinline__ void pin(T2* v) {
+#pragma unroll
+  for (int k = 0; k < N; ++k) { asm volatile("" : "+v"(v[k].x), "+v"(v[k].y)); }
+}
+// Element at a 32-bit byte offset from a uniform base: one VGPR of address per access (a state buffer
+// is below 4 GiB), where element pointers would hold two.
+template<bool NT> __device__ __forceinline__ T2 ldo(const T2* base, uint32_t bytes) {
+  return ldx<NT>((const T2*)((const char*)base + bytes));
+}
+template<bool NT> __device__ __forceinline__ void sto(T2* base, uint32_t bytes, T2 v) { stx<NT>((T2*)((char*)base + bytes), v); }
+
+// f on the part of v that an exchange of elements E moves in round p: v itself, or its real, then its imaginary part
+template<class E, class F> __device__ __forceinline__ void part(T2& v, int p, F f) {
+  if constexpr (std::is_same_v<E, double>) {
+    f(p ? v.y : v.x);
+  } else {
+    f(v);
+  }
+}
+// v of the lane 8 away in the row of 16 (DPP row rotate by 8)
+__device__ __forceinline__ double lane8(double v) {
+  const uint64_t x = __double_as_longlong(v);
+  const uint32_t lo = __builtin_amdgcn_mov_dpp((int)x, 0x128, 0xf, 0xf, true);
+  const uint32_t hi = __builtin_amdgcn_mov_dpp((int)(x >> 32), 0x128, 0xf, 0xf, true);
+  return __longlong_as_double((uint64_t)hi << 32 | lo);
+}
+__device__ __forceinline__ T2 lane8(T2 v) { return make_double2(lane8(v.x), lane8(v.y)); }
+
+// w^k for 1 <= k < 16 from the six exact powers w^1, w^2, w^3, w^4, w^8, w^12: at most one product.
+struct Pow16 {
+  T2 lo[3], hi[3];
+  __device__ __forceinline__ T2 operator()(int k) const {
+    if (k % 4 == 0) { return hi[k / 4 - 1]; }
+    if (k < 4) { return lo[k - 1]; }
+    return cmul(hi[k / 4 - 1], lo[k % 4 - 1]);
+  }
+};
+
+// Dft<R> with the sub-transforms of a composite R kept one after the other: left to itself the
+// scheduler interleaves them, and their temporaries spill.
+template<int R> struct Split {
+  static constexpr int P = 0, Q = 0;
+};
+template<> struct Split<15> { static constexpr int P = 3, Q = 5; };
+template<> struct Split<14> { static constexpr int P = 2, Q = 7; };
+template<> struct Split<12> { static constexpr int P = 4, Q = 3; };
+template<> struct Split<16> { static constexpr int P = 4, Q = 4; };
+template<int R, bool INV> __device__ __forceinline__ void dftSeq(T2* a) {
+  constexpr int P = Split<R>::P, Q = Split<R>::Q;
+  pin<R>(a);
+  if constexpr (P == 0) {
+    Dft<R, INV>::run(a);
+  } else {
+    T2 b[Q][P];
+#pragma unroll
+    for (int k2 = 0; k2 < Q; ++k2) {
+#pragma unroll
+      for (int k1 = 0; k1 < P; ++k1) { b[k2][k1] = a[Q * k1 + k2]; }
+      Dft<P, INV>::run(b[k2]);
+#pragma unroll
+      for (int m1 = 1; m1 < P; ++m1) { b[k2][m1] = rootMul<R, INV>(b[k2][m1], k2 * m1); }
+      pin<P>(b[k2]);
+    }
+#pragma unroll
+    for (int m1 = 0; m1 < P; ++m1) {
+      T2 c[Q];
+#pragma unroll
+      for (int k2 = 0; k2 < Q; ++k2) { c[k2] = b[k2][m1]; }
+      Dft<Q, INV>::run(c);
+      pin<Q>(c);
+#pragma unroll
+      for (int m2 = 0; m2 < Q; ++m2) { a[m1 + P * m2] = c[m2]; }
+    }
   }
 }
 
-// ---------------------------------------------------------------- column pass
-// MULTI = false: grid (W/2, batch), group q handles the column pair q; LDS: two
-// colRegionX<H>() regions (lx layout) and one twiddle table (colTwSize<H>() entries).
-// MULTI = true: grid (G, batch) with G <= W/2, group x handles the pairs x, x + G, x + 2G,
-// ... below W/2; LDS: the two regions and two tables. T threads; modes as k_col.
-// For H >= 2304 the root tables (colRootSlots<H>() entries) follow the twiddle table(s).
-// With several pairs per group, the next pair's column data and twiddle-table entries
-// are requested right after the current pair's first stage and stay in registers while
-// the current pair is transformed, squared and stored, so that HBM reads overlap the
-// LDS work instead of each group waiting for its loads with nothing else to do. The next
-// table goes to the other table buffer; a barrier at the end of each pair keeps the
-// regions and that buffer free until every wave is done with them.
-template<int H, int T, int C0, int C1, int C2, bool MULTI = false>
-__global__ __launch_bounds__(T) void k_colx(const JobDesc* __restrict__ jobs, int mode, int fi, int oi) {
-  static_assert(C0 * C1 * C2 == H && C0 == 16, "plan");
+// Grid (W/2, batch), T threads, LDS 2*colRegionX(H) doubles (the two columns) and ColTab::LDS twiddles; modes as k_col
+// (SQ: COL_SQUARE only, compiled alone because the other modes' registers would spill in it).
+template<int H, int T, int C0, int C1, int C2, bool SPLIT, bool NT, bool SQ>
+__global__ __launch_bounds__(T, SPLIT ? 4 : 2) void k_colx(const JobDesc* __restrict__ jobs, int modeArg, int fi, int oi) {
+  using L = ColTab<H, C0, C1, C2>;
+  static_assert(L::LDS == (int)colTabLds(H) && colRadices(H).c0 == C0 && colRadices(H).c2 == C2, "column table");
+  constexpr int REG = colRegionX(H, SPLIT);
+  using E = std::conditional_t<SPLIT, double, T2>;
+  constexpr int NB0 = H / C0, NB1 = H / C1, NB2 = H / C2, B = T / 2;
+  static_assert(C0 * C1 * C2 == H && NB0 <= B && NB1 <= B && NB2 <= B && (NB2 + 31) / 32 == T / 64 && B <= L::ROOTS, "plan");
+  constexpr int CM = C0 > C1 ? (C0 > C2 ? C0 : C2) : (C1 > C2 ? C1 : C2);
+  const int mode = SQ ? COL_SQUARE : modeArg;
   extern __shared__ T2 lds[];
-  constexpr int REG = colRegionX<H>();
-  constexpr int NB0 = H / C0;
-  constexpr int NBT = 2 * NB0;
-  constexpr int MB0 = (NBT + T - 1) / T;
-  constexpr int TWS = colTwSize<H>();
-  constexpr int MT = (TWS + T - 1) / T;
-  // exact root tables for two of the stages where LDS allows (one group per CU anyway)
-  constexpr bool ROOTS = H >= 2304;
-  T2* const roots = lds + 2 * REG + (MULTI ? 2 : 1) * TWS;
+  T2* const tab = lds + (SPLIT ? 1 : 2) * REG;
   const JobDesc& J = jobs[blockIdx.y];
   const int W = J.W, R = J.R, lgR = J.lgR;
-  const int tid0 = threadIdx.x;
-  // the column data streams through with non-temporal accesses from H = 768 up (at 512 x
-  // 256 the 2 MB buffers stay cached between passes and plain accesses measured faster)
-  constexpr bool NT = H >= 768;
+  // XCD x (group i runs on XCD i mod 8) takes the pairs x*W/16 ...: neighbouring pairs share a line
+  // block's 256-byte runs, which then go through one L2
+  const int q = (blockIdx.x & 7) * (W / 16) + (blockIdx.x >> 3);
+  // Column of the pair and butterfly: rows of 16 lanes alternate between the columns; in the middle (last forward,
+  // first inverse stage, names ending in P) runs of 8, so that the partner is in the same row.
+  const int h = (threadIdx.x >> 4) & 1, hP = (threadIdx.x >> 3) & 1;
+  int j = (threadIdx.x >> 5) * 16 + (threadIdx.x & 15), jP = (threadIdx.x >> 4) * 8 + (threadIdx.x & 7);
+  E* const reg = reinterpret_cast<E*>(lds) + h * REG;  // the column's region
+  E* const regP = reinterpret_cast<E*>(lds) + hP * REG;
   T2* io = J.freq[fi];
   const T2* other = (mode == COL_MUL) ? J.freq[oi] : nullptr;
-  const size_t blockStride = (size_t)W * R;
-  const int per = 2 * R;
-  // Element (line l, column h of pair q) lies at offset (l/R)*W*R + 2qR + hR + l%R, below ND < 2^32.
-  // The host runs this pass only when R divides H/16 = NB0, so for the lines l = j + k*NB0 of a
-  // stage-0 butterfly the offset is off(j) + k*kStride: one add per element.
-  const uint32_t kStride = (uint32_t)(NB0 >> lgR) * (uint32_t)(W * R);
-  auto offset0 = [&](int q, int h, int j) -> uint32_t {
-    return (uint32_t)(j >> lgR) * (uint32_t)(W * R) + (uint32_t)(2 * q * R + (h << lgR) + (j & (R - 1)));
+  const uint32_t WR = (uint32_t)(W * R), colBase = (uint32_t)(2 * q * R);
+  // line l of column c lies at element spos(c, l); line j + k*NB0 at spos(h, j) + k*kStride/16 (the host runs this
+  // pass only when R divides NB0)
+  const uint32_t kStride = (uint32_t)(NB0 >> lgR) * WR * 16;
+  auto spos = [&](int c, int l) -> uint32_t {
+    return (uint32_t)(l >> lgR) * WR + colBase + (uint32_t)(c << lgR) + (uint32_t)(l & (R - 1));
+  };
+  // Mid twiddle of line j + k*NB0: base * S[k], the S entries uniform. For q = 0 column 0 has none and column W/2
+  // its own; the latter pairs with itself, so it is not conjugated.
+  const int a = q ? q : W / 2;
+  const double sgn = (q && h) ? -1.0 : 1.0;
+  auto midBase = [&](int l) -> T2 { return cmul(gld(J.twMidA + a * 64 + (l & 63)), gld(J.twMidB + a * J.nHi + (l >> 6))); };
+  auto mid = [&](T2 base, int k) -> T2 {
+    const CONSTANT double* s = (const CONSTANT double*)(J.twMidM + a * 16 + k);
+    T2 w = k ? cmul(base, make_double2(s[0], s[1])) : base;
+    if (!q) {
+      asm volatile("");  // a branch that all other groups skip, not selects in every group
+      if (!h) { w = make_double2(1, 0); }
+    }
+    return w;
+  };
+  auto loadWt = [&](Pow16& wt, int t0) {  // w_H^(j*k)
+    const T2* t = J.colTab + L::LDS + t0;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      wt.lo[k] = gld(t + k * L::ROOTS);
+      wt.hi[k] = gld(t + (3 + k) * L::ROOTS);
+    }
   };
 
-  // Lane order within 2R lanes: (column h, line-in-block r), so 2R lanes read 2R*16
-  // contiguous bytes of one line block.
-  T2 xin[MB0][C0];
-  auto loadPair = [&](int q, int tid) {
-#pragma unroll
-    for (int m = 0; m < MB0; ++m) {
-      const int g = tid + m * T;
-      if (NBT % T == 0 || g < NBT) {
-        const int h = (g >> lgR) & 1;
-        const int j = ((g >> (lgR + 1)) << lgR) | (g & (R - 1));
-        const uint32_t o = offset0(q, h, j);
-#pragma unroll
-        for (int k = 0; k < C0; ++k) { xin[m][k] = ldx<NT>(io + (o + k * kStride)); }
-      }
-    }
-  };
+  constexpr std::integral_constant<int, C0> c0;
+  constexpr std::integral_constant<int, C1> c1;
+  constexpr std::integral_constant<int, C2> c2;
+  // A stage with NB < T/2 butterflies runs in the waves that have one (uniform branches); the lanes past NB in
+  // the last of them repeat butterfly NB - 1 (same addresses, same values).
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  auto runs = [&](int nb) -> bool { return nb == B || wave < (nb + 31) / 32; };
+  auto bf = [&](int nb) -> int { return nb % 32 == 0 ? j : min(j, nb - 1); };
+  if (NB2 % 32) { jP = min(jP, NB2 - 1); }
 
-  int q = blockIdx.x;
-  // the column data is requested before the twiddle table is filled, so the two latencies overlap
-  loadPair(q, tid0);
-  fillColTw<H>(J, lds + 2 * REG, q, q ? W - q : W / 2, tid0, T);
-  if constexpr (ROOTS) { fillColRoots<H>(J, roots, tid0, T); }
-  __syncthreads();
-  for (int it = 0;; ++it) {
-    // a fresh copy of the thread index per pair: offsets derived from it are recomputed
-    // in each pair instead of being hoisted out of the loop and held in registers
-    int tid = tid0;
-    if constexpr (MULTI) { asm volatile("" : "+v"(tid)); }
-    const ColTw<H, ROOTS> tw{lds + 2 * REG + (it & 1) * TWS, roots};
-    const int a0 = q, a1 = q ? W - q : W / 2;
-    const size_t colBase = (size_t)2 * q * R;
-    const T2 wa = gld(J.twPair + (q ? a0 : a1));  // column a0's pairing twiddle, or column W/2's for q = 0
-    const int qn = MULTI ? q + (int)gridDim.x : W / 2;
-
-    // forward stage 0 (radix C0, Ns = 1), fused with the load and the mid twiddle
+  T2 x[CM];
+  // One exchange: nw butterflies write x[k], k < n, at w + k*ws, nr butterflies read x[k], k < m, at r + k*rs; real
+  // parts, then imaginary parts.
+  auto exchange = [&](auto n, int nw, E* w, int ws, auto m, int nr, const E* r, int rs) {
 #pragma unroll
-    for (int m = 0; m < MB0; ++m) {
-      const int g = tid + m * T;
-      if (NBT % T == 0 || g < NBT) {
-        const int h = (g >> lgR) & 1;
-        const int j = ((g >> (lgR + 1)) << lgR) | (g & (R - 1));
-        const T2 base = tw.mid(h, j);
-        T2 v[C0];
+    for (int p = 0; p < (SPLIT ? 2 : 1); ++p) {
+      __syncthreads();
+      if (runs(nw)) {
 #pragma unroll
-        for (int k = 0; k < C0; ++k) { v[k] = cmul(xin[m][k], k ? cmul(base, tw.s(h, k)) : base); }
-        Dft<C0, false>::run(v);
-#pragma unroll
-        for (int k = 0; k < C0; ++k) { lds[h * REG + (lx(j * C0) ^ k)] = v[k]; }
-      }
-    }
-    // prefetch of the next pair: table entries first (written to LDS below, so their wait
-    // does not cover the column data), then the column data
-    T2 twn[MT];
-    if (MULTI && qn < W / 2) {
-#pragma unroll
-      for (int m = 0; m < MT; ++m) {
-        const int i = tid + m * T;
-        if (TWS % T == 0 || i < TWS) { twn[m] = colTwEntry<H>(J, i, qn, W - qn); }
-      }
-      loadPair(qn, tid);
-    }
-    __syncthreads();
-    XStages<H, REG, 2, T, false, false, true, C0, C1, C2>::run(lds, tw, tid);
-    if (MULTI && qn < W / 2) {
-      T2* tabn = lds + 2 * REG + ((it + 1) & 1) * TWS;
-#pragma unroll
-      for (int m = 0; m < MT; ++m) {
-        const int i = tid + m * T;
-        if (TWS % T == 0 || i < TWS) { tabn[i] = twn[m]; }
-      }
-    }
-
-    if (mode == COL_FWD) {
-      for (int e = tid; e < 2 * H; e += T) {
-        int lb = e / per;
-        int wi = e - lb * per;
-        int h = wi >> lgR;
-        int b = lb * R + (wi & (R - 1));
-        stx<NT>(io + (size_t)lb * blockStride + colBase + wi, lds[h * REG + lx(b)]);
-      }
-    } else {
-      auto spos = [&](int h, int b) -> size_t { return (size_t)(b >> lgR) * blockStride + colBase + (h << lgR) + (b & (R - 1)); };
-      if (q) {
-        for (int b = tid; b < H; b += T) {
-          int bp = H - 1 - b;
-          T2 X = lds[lx(b)], Xp = lds[REG + lx(bp)];
-          T2 w = cmul(wa, tw(b));
-          if (other) {
-            pairMul(X, Xp, gld(other + spos(0, b)), gld(other + spos(1, bp)), w);
-          } else {
-            pairSq(X, Xp, w);
-          }
-          lds[lx(b)] = X;
-          lds[REG + lx(bp)] = Xp;
-        }
-      } else {
-        for (int i = tid; i <= H; i += T) {
-          if (i <= H / 2) {
-            int b = i, bp = (H - i) % H;
-            T2 X = lds[lx(b)], Xp = lds[lx(bp)];
-            T2 w = tw(b);
-            if (other) {
-              pairMul(X, Xp, gld(other + spos(0, b)), gld(other + spos(0, bp)), w);
-            } else {
-              pairSq(X, Xp, w);
-            }
-            lds[lx(b)] = X;
-            if (bp != b) { lds[lx(bp)] = Xp; }
-          } else {
-            int b = i - H / 2 - 1, bp = H - 1 - b;
-            T2 X = lds[REG + lx(b)], Xp = lds[REG + lx(bp)];
-            T2 w = cmul(wa, tw(b));
-            if (other) {
-              pairMul(X, Xp, gld(other + spos(1, b)), gld(other + spos(1, bp)), w);
-            } else {
-              pairSq(X, Xp, w);
-            }
-            lds[REG + lx(b)] = X;
-            lds[REG + lx(bp)] = Xp;
-          }
-        }
+        for (int k = 0; k < n; ++k) { part<E>(x[k], p, [&](auto& e) { w[k * ws] = e; }); }
       }
       __syncthreads();
-      // inverse stages radix C1 then C2 (the reverse of the forward order would put the radix-C2
-      // stage first, whose stride-C2 writes hit few LDS banks for C2 = 15)
-      XStages<H, REG, 2, T, true, false, true, 1, C1, C2>::run(lds, tw, tid);
-
-      // last inverse stage (radix C0, Ns = NB0), fused with the conjugate mid twiddle and the store
+      if (runs(nr)) {
 #pragma unroll
-      for (int m = 0; m < MB0; ++m) {
-        const int g = tid + m * T;
-        if (NBT % T == 0 || g < NBT) {
-          const int h = (g >> lgR) & 1;
-          const int j = ((g >> (lgR + 1)) << lgR) | (g & (R - 1));
-          T2 v[C0];
-#pragma unroll
-          for (int k = 0; k < C0; ++k) { v[k] = lds[h * REG + lx(j + k * NB0)]; }
-#pragma unroll
-          for (int k = 1; k < C0; ++k) { v[k] = cmulc(v[k], tw.pk(j, k)); }
-          Dft<C0, true>::run(v);
-          const T2 base = tw.mid(h, j);
-          const uint32_t o = offset0(q, h, j);
-#pragma unroll
-          for (int k = 0; k < C0; ++k) { stx<NT>(io + (o + k * kStride), cmulc(v[k], k ? cmul(base, tw.s(h, k)) : base)); }
-        }
+        for (int k = 0; k < m; ++k) { part<E>(x[k], p, [&](auto& e) { e = r[k * rs]; }); }
       }
     }
-    if (!MULTI || qn >= W / 2) { break; }
+  };
+  for (int i = threadIdx.x; i < L::LDS; i += T) { tab[i] = gld(J.colTab + i); }
+  if (runs(NB0)) {
+    const int j0 = bf(NB0);
+    const uint32_t o = spos(h, j0) * 16;
+#pragma unroll
+    for (int k = 0; k < C0; ++k) { x[k] = ldo<NT>(io, o + k * kStride); }
+    const T2 base = midBase(j0);
+#pragma unroll
+    for (int k = 0; k < C0; ++k) {
+      x[k] = cmul(make_double2(x[k].x, sgn * x[k].y), mid(base, k));
+      pin<1>(&x[k]);
+    }
+    dftSeq<C0, false>(x);
+  }
+  FRESH(j);
+  // stage 1: radix C1, Ns = C0
+  {  // rows of C0 | 1; NB1 is a multiple of C0
+    const int j1 = bf(NB1);
+    constexpr int PAD = (C0 | 1) - C0;
+    exchange(c0, NB0, reg + bf(NB0) * (C0 | 1), 1, c1, NB1, reg + j1 + j1 / C0 * PAD, NB1 + NB1 / C0 * PAD);
+  }
+  if (runs(NB1)) {
+    const T2* t = tab + L::A + (bf(NB1) % C0) * L::KS - 1;
+#pragma unroll
+    for (int k = 1; k < C1; ++k) {
+      x[k] = cmul(x[k], t[k]);
+      pin<1>(&x[k]);
+    }
+    dftSeq<C1, false>(x);
+  }
+  FRESH(j);
+  // stage 2: radix C2, Ns = C0*C1 = NB2: bins j + k*NB2
+  Pow16 wt;
+  loadWt(wt, jP);
+  {  // blocks of C0*C1 = NB2 elements, C0 further apart
+    const int j1 = bf(NB1), blk = j1 / C0;
+    exchange(c1, NB1, reg + j1 + blk * NB2, C0, c2, NB2, regP + jP, NB2 + C0);
+  }
+  T2 wb = wt.lo[0];
+#pragma unroll
+  for (int k = 1; k < C2; ++k) {
+    x[k] = cmul(x[k], wt(k));
+    pin<1>(&x[k]);
+  }
+  dftSeq<C2, false>(x);
+  pin<C2>(x);
+  FRESH(jP);
+
+  if (mode == COL_FWD) {  // the plain spectrum: column W - a's bin H-1-b is conj(x[k])
+#pragma unroll
+    for (int k = 0; k < C2; ++k) {
+      const int b = jP + k * NB2;
+      stx<false>(io + spos(hP, q && hP ? H - 1 - b : b), q && hP ? conj2(x[k]) : x[k]);
+    }
+    return;
+  }
+
+  // pairing, with P = conj(partner): X <- X*Y - (1 + w)(X - P)(Y - Q)/4, where Y, Q are the second operand's bins
+  // (X, P themselves when squaring); w of bin b is w_ND^(a + W*b). P is in the lane 8 away; for q = 0 columns 0 (b
+  // pairs with -b) and W/2 (b with H-1-b) pair within themselves: bin j + k*NB2 with bin (NB2 - j or NB2 - 1 - j) +
+  // (C2-1-k)*NB2, through LDS two registers at a time (j = 0 of column 0: bin k*NB2 with (C2-k)*NB2, kept apart).
+  wb = cscale(cmul(gld(J.twPair + (q || hP ? a : 0)), wb), 0.25);
+  T2* const self = lds + 2 * T;
+  if (!q) {
     __syncthreads();
-    q = qn;
+    if (threadIdx.x == 0) {
+#pragma unroll
+      for (int k = 0; k < C2; ++k) { self[k] = x[k]; }
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < (C2 + 1) / 2; ++k) {
+    const int k2 = C2 - 1 - k;
+    T2 P, P2;
+    if (q) {
+      P = lane8(x[k]);
+      P2 = lane8(x[k2]);
+    } else {
+      T2* buf = lds + hP * B;
+      __syncthreads();
+      buf[jP] = x[k];
+      buf[T + jP] = x[k2];
+      __syncthreads();
+      const int jm = hP ? NB2 - 1 - jP : NB2 - jP;
+      const bool own = jm == NB2;
+      P = conj2(*(own ? self + (k ? C2 - k : 0) : buf + T + jm));
+      P2 = conj2(*(own ? self + (C2 - k2) : buf + jm));
+    }
+#pragma unroll
+    for (int i = 0; i < (k == k2 ? 1 : 2); ++i) {
+      const int kk = i ? k2 : k;
+      pin<1>(&wb);
+      const T2 w = rootMul<C2, false>(wb, kk);
+      const T2 v = make_double2(0.25 + w.x, w.y);
+      const T2 D = csub(x[kk], i ? P2 : P);
+      if (SQ || !other) {
+        x[kk] = csub(csqr(x[kk]), cmul(v, csqr(D)));
+      } else {
+        const int b = jP + kk * NB2;
+        T2 Y, Q;
+        if (q) {
+          Y = gld(other + spos(hP, hP ? H - 1 - b : b));
+          if (hP) { Y.y = -Y.y; }
+          Q = lane8(Y);
+        } else {
+          Y = gld(other + spos(hP, b));
+          Q = conj2(gld(other + spos(hP, hP ? H - 1 - b : b ? H - b : 0)));
+        }
+        x[kk] = csub(cmul(x[kk], Y), cmul(v, cmul(D, csub(Y, Q))));
+      }
+      pin<1>(&x[kk]);
+    }
+  }
+  FRESH(jP);
+
+  // inverse stage 0: radix C2, Ns = 1, butterfly jP: the registers
+  dftSeq<C2, true>(x);
+  // stage 1: radix C1, Ns = C2
+  FRESH(j);
+  {  // rows of C2 | 1; NB1 is a multiple of C2
+    const int j1 = bf(NB1);
+    constexpr int PAD = (C2 | 1) - C2;
+    exchange(c2, NB2, regP + jP * (C2 | 1), 1, c1, NB1, reg + j1 + j1 / C2 * PAD, NB1 + NB1 / C2 * PAD);
+  }
+  if (runs(NB1)) {
+    const T2* t = tab + L::B + (bf(NB1) % C2) * L::KS - 1;
+#pragma unroll
+    for (int k = 1; k < C1; ++k) {
+      x[k] = cmulc(x[k], t[k]);
+      pin<1>(&x[k]);
+    }
+    dftSeq<C1, true>(x);
+  }
+  FRESH(j);
+  // stage 2: radix C0, Ns = NB0, then the conjugate mid twiddle and the store
+  const int j0 = bf(NB0);
+  loadWt(wt, j0);
+  {  // blocks of C1*C2 = NB0 elements, C2 further apart
+    const int j1 = bf(NB1), blk = j1 / C2;
+    exchange(c1, NB1, reg + j1 + blk * NB0, C2, c0, NB0, reg + j0, NB0 + C2);
+  }
+  if (runs(NB0)) {
+#pragma unroll
+    for (int k = 1; k < C0; ++k) {
+      x[k] = cmulc(x[k], wt(k));
+      pin<1>(&x[k]);
+    }
+    dftSeq<C0, true>(x);
+    pin<C0>(x);
+    FRESH(j);
+    const T2 base = midBase(bf(NB0));
+    const uint32_t o = spos(h, bf(NB0)) * 16;
+#pragma unroll
+    for (int k = 0; k < C0; ++k) {
+      const T2 y = cmulc(x[k], mid(base, k));
+      sto<NT>(io, o + k * kStride, make_double2(y.x, sgn * y.y));
+    }
   }
 }
 
 // ---------------------------------------------------------------- column pass, one region
-// The two columns of the pair go through one LDS region in turn (half the LDS of k_colx,
-// so two groups share a CU), and the real-signal pairing runs in registers: the last
+// The two columns of the pair go through one LDS region in turn, and the real-signal pairing runs in registers: the last
 // forward stage (radix C2, T = H/C2 butterflies) leaves thread t holding X0[t + T*k];
 // column 1's last stage is computed for butterfly T-1-t, so the partner of X0[b],
 // X1[H-1-b], is X1[(T-1-t) + T*(C2-1-k)] in the same thread. The inverse's first stage
@@ -606,7 +671,7 @@ __global__ __launch_bounds__(H / C2, 2) void k_coly(const JobDesc* __restrict__ 
       for (int k = 0; k < C0; ++k) { lds[padi(j * C0 + k)] = v[k]; }
     }
     __syncthreads();
-    XStages<H, REG, 1, T, false, false, false, C0, C1>::run(lds, tw, tid);
+    XStages<H, REG, 1, T, false, false, C0, C1>::run(lds, tw, tid);
 #pragma unroll
     for (int k = 0; k < C2; ++k) { out[k] = lds[padi(jl + k * T)]; }
 #pragma unroll
@@ -621,7 +686,7 @@ __global__ __launch_bounds__(H / C2, 2) void k_coly(const JobDesc* __restrict__ 
 #pragma unroll
     for (int k = 0; k < C2; ++k) { lds[padi(jl * C2 + k)] = in[k]; }
     __syncthreads();
-    XStages<H, REG, 1, T, true, false, false, C2, C1>::run(lds, tw, tid);
+    XStages<H, REG, 1, T, true, false, C2, C1>::run(lds, tw, tid);
     if (tid < NB0) {
       const int j = tid;
       T2 v[C0];
@@ -701,7 +766,6 @@ __global__ __launch_bounds__(H / C2, 2) void k_coly(const JobDesc* __restrict__ 
 // Weight data of one line read through the scalar cache: the line index is uniform across the
 // group (readfirstlane), so the loads are scalar and the values live in SGPRs. Vector loads of
 // them would also sit in the in-order vector memory counter behind a prefetch still in flight.
-#define CONSTANT __attribute__((address_space(4)))
 struct LineWs {
   double w0, w1, iw0, iw1;
   uint32_t e0, e1;
@@ -867,7 +931,7 @@ template<int W, int R, int F0, int F1, int F2> struct RowPass {
   }
   // inverse W-point FFT of the R lines (LDS stages, then the radix-F0 stage into registers)
   __device__ __forceinline__ static void inverse(T2* lds, const Tw& tw, int tid, int cb, T2 (&v)[R][F0]) {
-    XStages<W, REG, R, T, true, true, false, 1, F2, F1>::run(lds, tw, tid);
+    XStages<W, REG, R, T, true, true, 1, F2, F1>::run(lds, tw, tid);
     __syncthreads();
     // last inverse stage (radix F0, Ns = T): butterfly cb of each line -> columns cb + k*T
 #pragma unroll
@@ -975,7 +1039,7 @@ template<int W, int R, int F0, int F1, int F2> struct RowPass {
       for (int k = 0; k < F0; ++k) { lds[r * REG + padi(cb * F0 + k)] = v[r][k]; }
     }
     __syncthreads();
-    XStages<W, REG, R, T, false, true, false, F0, F1, F2>::run(lds, tw, tid);
+    XStages<W, REG, R, T, false, true, F0, F1, F2>::run(lds, tw, tid);
     __syncthreads();
   }
   // the block from the line regions, slot order

@@ -66,9 +66,9 @@ int owl_fft_tune_entry(uint32_t i, double* cost, char* spec, size_t specLen, uin
  * flags: OWL_LONG_CARRY = full carry every iteration (the reference's -carry long);
  *        OWL_GENERIC = runtime-plan kernels even where a shape-specialized pass exists;
  *        OWL_COL_ONE_REGION = the column pass variant that takes the two columns through one
- *        LDS region in turn (pairing in registers) where the two-region pass exists;
- *        OWL_COL_ONE_PAIR = the two-region column pass with one column pair per group where
- *        the variant with two pairs per group would be chosen. */
+ *        LDS region in turn where the pass that keeps a butterfly of both in registers exists;
+ *        OWL_COL_ONE_PAIR = the latter with one column pair on a CU at a time (exchanges of complex
+ *        elements) where its split variant, with two pairs per CU, would be chosen. */
 enum { OWL_LONG_CARRY = 1, OWL_GENERIC = 2, OWL_COL_ONE_REGION = 4, OWL_COL_ONE_PAIR = 8 };
 int owl_gpu_create(uint32_t E, const char* spec, int flags, uint32_t lineBlock, owl_gpu* gpu);
 int owl_gpu_destroy(owl_gpu gpu);
