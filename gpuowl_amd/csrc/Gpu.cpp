@@ -163,6 +163,14 @@ Gpu::Gpu(u32 E, const FFTConfig& fftIn, const GpuOptions& optIn) : E{E}, fft{fft
     // twiddle tables (W >= 512)
     rowLds = R * (W + W / 16 + ((R == 4 || R == 8) ? 6 : 4)) * 16 + 64 +
              (W >= 1024 ? (rowT + 240 + W / 16) * 16 : W >= 512 ? (132 + rowT) * 16 : 0);
+    // k_rowm: its own LDS layout, with complex and with split exchanges (coltab.h)
+    const std::string wr = std::to_string(W) + "r" + std::to_string(R);
+    if (haveKernel("rowcp" + wr)) {
+      rowM = true;
+      const u32 F0 = W / rowT, F1 = W / (16 * F0);
+      rowLds = 16 * rowLayout(W, R, F0, F1, false).slots;
+      rowLdsS = 16 * rowLayout(W, R, F0, F1, true).slots;
+    }
   } else {
     rowKernel = "row" + std::to_string(rowT);
   }
@@ -188,7 +196,7 @@ Gpu::Gpu(u32 E, const FFTConfig& fftIn, const GpuOptions& optIn) : E{E}, fft{fft
   // ---- tables: twiddles shared per shape (TrigBufCache), weights per exponent (long double, rounded once)
   const u32 step = stepOf(N, E);
   const u32 nHi = (H + 63) / 64;
-  trig_ = TrigBufCache::get(W, H, queue_);
+  trig_ = TrigBufCache::get(W, H, useY, queue_);
   std::vector<LineW> lineW(H);
   for (u32 l = 0; l < H; ++l) {
     for (u32 rep = 0; rep < 2; ++rep) {
@@ -241,8 +249,9 @@ Gpu::Gpu(u32 E, const FFTConfig& fftIn, const GpuOptions& optIn) : E{E}, fft{fft
     // Per row-pass thread and block: which of its words are big and which weight exponents wrap
     // (the tests of wordWeight, src/Gpu.cpp:40-127's bitsCF), so the pass does not recompute them.
     const u32 T = rowT, F0 = W / T;
-    // thread tid's columns are colBase(tid) + k*T (RowPass::colBase, kfixed.h)
-    auto colBase = [F0](u32 tid) -> u32 {
+    // thread tid's columns are colBase(tid) + k*T (RowPass::colBase, kfixed.h; tid + k*T in k_rowm)
+    auto colBase = [F0, this](u32 tid) -> u32 {
+      if (rowM) { return tid; }
       const u32 b = tid & 15, hi = tid & ~15u;
       if (F0 == 2) { return hi | (b & 3) | ((b >> 3) << 2) | (((b >> 2) & 1) << 3); }
       if (F0 == 4) { return hi | (b & 1) | (((b >> 3) & 1) << 1) | (((b >> 1) & 3) << 2); }
@@ -290,6 +299,13 @@ Gpu::Gpu(u32 E, const FFTConfig& fftIn, const GpuOptions& optIn) : E{E}, fft{fft
   jobs_.write(queue_, {J});
 
   kRow = Kernel(rowKernel);
+  if (rowM) {
+    const std::string wr = rowKernel.substr(4);
+    kRowF[0][0] = Kernel("rowcp" + wr);
+    kRowF[0][1] = Kernel("rowcn" + wr);
+    kRowF[1][0] = Kernel("rowsp" + wr);
+    kRowF[1][1] = Kernel("rowsn" + wr);
+  }
   colOne_ = colKernel;
   kCol = Kernel(colOne_);
   if (colX_) {
@@ -409,8 +425,10 @@ void Gpu::rowFused(bool ll, u32 roeSlot, Launch L) {
   // the runtime-plan k_row: nb + 1 groups in start-ticket order
   int mode = ROW_FUSED, fi = 0, wi = 0, opts = (ll ? 1 : 0) | (rowChunked ? 4 : 0);
   u32 tag = nextStairTag();
-  kRow(L.q, rowChunked ? 8 * ((nb + 7) / 8 + 1) : nb + 1, L.n, rowT, rowLds,
-       {&L.jobs, &mode, &fi, &wi, &opts, &roeSlot, &tag});
+  const u32 groups = rowChunked ? 8 * ((nb + 7) / 8 + 1) : nb + 1;
+  const bool split = rowM && rowSplit(L.n);
+  const Kernel& k = rowM ? kRowF[split][streamed(L.n)] : kRow;
+  k(L.q, groups, L.n, rowT, split ? rowLdsS : rowLds, {&L.jobs, &mode, &fi, &wi, &opts, &roeSlot, &tag});
 }
 
 void Gpu::rowLeadInTo(Buf in, int freqIdx, Launch L) {
@@ -431,7 +449,7 @@ void Gpu::carryAll(Buf b, Launch L) {
   kCarryFix(L.q, 1, L.n, 256, 0, {&L.jobs, &wi, &co});
 }
 
-// Whether a column launch of nJobs jobs streams the state with non-temporal accesses: when the states together fit the
+// Whether a launch of nJobs jobs streams the state with non-temporal accesses: when the states together fit the
 // L2s (which then write back early instead of at the end of the launch) and when they exceed the 256 MB
 // Infinity Cache. Between, and below 6 MB, plain accesses are faster. Measured, us per squaring,
 // non-temporal / plain: 2 MB 16.4 / 15.7, 9.4 MB 31.2 / 33.8, 25 MB 37.0 / 40.1, 42 MB 56.3 / 57.9, 50 MB 64.8 / 65.2,
@@ -441,8 +459,12 @@ bool Gpu::streamed(u32 nJobs) const {
   return bytes >= (6u << 20) && (bytes <= (56u << 20) || bytes > (256u << 20));
 }
 
-// Whether a squaring column launch of nJobs jobs exchanges real and imaginary parts one after the other (four
-// waves per SIMD), compiled from H = 2304 up, where a group with complex exchanges takes
+// Whether a fused row launch of nJobs jobs exchanges real and imaginary parts one after the other (four waves per
+// SIMD): when it has more waves than the complex exchange keeps on the device (two per SIMD). Measured, us per row
+// launch, split / complex: 1024 x 3840 38.7 / 41.7, 1024 x 1536 25.2 / 22.5; batches 256 x 1024 x 64 jobs 150 / 160.
+bool Gpu::rowSplit(u32 nJobs) const { return u64(nb) * nJobs * (rowT / 64) > 8 * cus_; }
+
+// The same choice for the column pass, which has it from H = 2304 up, where a group with complex exchanges takes
 // more than half of a CU's LDS: when the pairs give every CU two groups. (us per launch, split / complex:
 // 1024 x 3840 38.4 / 47.4, 256 x 2304 19.1 / 18.7. Below 2304 the complex exchange is faster in batches too.)
 bool Gpu::colSplit(u32 nJobs) const { return haveSplit && u64(W / 2) * nJobs >= 2 * cus_; }

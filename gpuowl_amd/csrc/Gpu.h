@@ -84,10 +84,11 @@ public:
   u32 N, ND, W, H, R, nb, rowT, colT, rowLds, colLds;
   std::string rowKernel, colKernel;  // colKernel: what a launch of this job alone runs
   bool rowChunked = false;           // fused row launches in chunked per-XCD block order (nb >= 8)
-  // Variants of the squaring's column pass, chosen per launch by its number of jobs: exchanges of real and imaginary
+  // Variants of the squaring's passes, chosen per launch by its number of jobs: exchanges of real and imaginary
   // parts one after the other (split) or of complex elements, plain or non-temporal (streamed) accesses.
-  bool haveSplit = false;
-  u32 colSplitLds = 0;  // LDS bytes of the split variant
+  bool rowM = false, haveSplit = false;  // the row pass is k_rowm; the column pass has a split variant
+  u32 rowLdsS = 0, colSplitLds = 0;      // LDS bytes of the split variants
+  bool rowSplit(u32 nJobs) const;
   bool colSplit(u32 nJobs) const;
   bool streamed(u32 nJobs) const;
   std::string colKernelFor(u32 nJobs) const;  // the column kernel a launch of nJobs jobs runs
@@ -233,7 +234,7 @@ private:
   std::string colOne_;  // the column kernel without its "m" (split) suffix
   bool colX_ = false;   // the column pass is k_colx
   u32 cus_ = 1;         // compute units
-  Kernel kColSq[2][2];  // [split][streamed]: squaring column pass (colX_)
+  Kernel kRowF[2][2], kColSq[2][2];  // [split][streamed]: fused row pass (rowM), squaring column pass (colX_)
   Kernel kRow, kCol, kCarryB, kCarryFix, kWordsIn, kWordsOut, kResidue, kIsEqual, kSum64, kCopy;
 
   template<typename T> T* alloc(size_t n);

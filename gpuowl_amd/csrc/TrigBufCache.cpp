@@ -5,6 +5,7 @@
 
 #include <map>
 #include <mutex>
+#include <tuple>
 #include <vector>
 
 namespace {
@@ -31,24 +32,23 @@ std::vector<double2> colTabOf(u32 H) {
 }
 }  // namespace
 
-std::shared_ptr<const TrigTables> TrigBufCache::get(u32 W, u32 H, owl_queue q) {
+std::shared_ptr<const TrigTables> TrigBufCache::get(u32 W, u32 H, bool oneRegion, owl_queue q) {
   static std::mutex mtx;
-  static std::map<std::pair<u32, u32>, std::weak_ptr<const TrigTables>> cache;
+  static std::map<std::tuple<u32, u32, bool>, std::weak_ptr<const TrigTables>> cache;
   std::lock_guard<std::mutex> lock(mtx);
-  auto key = std::make_pair(W, H);
+  auto key = std::make_tuple(W, H, oneRegion);
   if (auto it = cache.find(key); it != cache.end()) {
     if (auto sp = it->second.lock()) { return sp; }
   }
   const u32 ND = W * H;
   const u32 nHi = (H + 63) / 64;
-  std::vector<double2> row(W), col(H), midA(size_t(W) * 64), midB(size_t(W) * nHi), pair(W), midS(size_t(W) * 16);
+  std::vector<double2> row(W), col(H), midA(size_t(W) * 64), midB(size_t(W) * nHi), pair(W), mid(size_t(W) * 16);
   for (u32 m = 0; m < W; ++m) { row[m] = d2(root1(W, m)); }
   for (u32 m = 0; m < H; ++m) { col[m] = d2(root1(H, m)); }
   for (u32 a = 0; a < W; ++a) {
     pair[a] = d2(root1(ND, a));
     for (u32 lo = 0; lo < 64; ++lo) { midA[size_t(a) * 64 + lo] = d2(root1(ND, u64(a) * lo)); }
     for (u32 hi = 0; hi < nHi; ++hi) { midB[size_t(a) * nHi + hi] = d2(root1(ND, u64(a) * 64 * hi % ND)); }
-    for (u32 k = 0; k < 16; ++k) { midS[size_t(a) * 16 + k] = d2(root1(ND, u64(a) * k * (H / 16) % ND)); }
   }
   auto t = std::make_shared<TrigTables>();
   t->row = Buffer<double2>(q, row);
@@ -56,14 +56,13 @@ std::shared_ptr<const TrigTables> TrigBufCache::get(u32 W, u32 H, owl_queue q) {
   t->midA = Buffer<double2>(q, midA);
   t->midB = Buffer<double2>(q, midB);
   t->pair = Buffer<double2>(q, pair);
-  t->midS = Buffer<double2>(q, midS);
-  if (const u32 c0 = colRadices(H).c0) {
-    std::vector<double2> midM(size_t(W) * 16);
+  const u32 c0 = oneRegion ? 16 : colRadices(H).c0;
+  if (c0) {
     for (u32 a = 0; a < W; ++a) {
-      for (u32 k = 0; k < 16; ++k) { midM[size_t(a) * 16 + k] = d2(root1(ND, u64(a) * k * (H / c0) % ND)); }
+      for (u32 k = 0; k < 16; ++k) { mid[size_t(a) * 16 + k] = d2(root1(ND, u64(a) * k * (H / c0) % ND)); }
     }
-    t->midM = Buffer<double2>(q, midM);
-    t->colTab = Buffer<double2>(q, colTabOf(H));
+    (oneRegion ? t->midS : t->midM) = Buffer<double2>(q, mid);
+    if (!oneRegion) { t->colTab = Buffer<double2>(q, colTabOf(H)); }
   }
   cache[key] = t;
   return t;

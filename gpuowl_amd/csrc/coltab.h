@@ -61,3 +61,24 @@ constexpr int colThreadsX(int H) {
   const int c = r.c0 < r.c1 ? (r.c0 < r.c2 ? r.c0 : r.c2) : (r.c1 < r.c2 ? r.c1 : r.c2);
   return (2 * (H / c) + 63) / 64 * 64;
 }
+
+// Row pass with 16 elements per thread (k_rowm): line strides of its exchanges in elements, and its LDS. Split
+// exchanges move doubles (real, then imaginary parts), the others complex elements.
+struct RowLayout {
+  int l1, l3, l4;  // exchanges 1, 3 and 4 (exchange 2: W)
+  int tab;         // 16-byte slots before the product table of 16 rows of ks entries
+  int ks, slots;   // slots: all of it, the 64 bytes of round-off values at the end included
+};
+constexpr int leastMod(int n, int r, int m) { return n + ((r - n) % m + m) % m; }  // least value >= n that is r mod m
+constexpr RowLayout rowLayout(int W, int R, int F0, int F1, bool split) {
+  RowLayout g{};
+  const int u = split ? 16 : 8;  // elements per LDS write cycle; a read serves twice as many
+  g.l1 = leastMod(W + W / 16, u / R, u);
+  g.l3 = W + W / 16;
+  g.l4 = leastMod(W + 16 * F0, 2 * u / R, 2 * u);
+  const int l = g.l1 > g.l4 ? (g.l1 > g.l3 ? g.l1 : g.l3) : (g.l4 > g.l3 ? g.l4 : g.l3);
+  g.ks = (F1 - 1) | 1;
+  g.tab = split ? (R * l + 1) / 2 : R * l;
+  g.slots = g.tab + 16 * g.ks + 4;
+  return g;
+}

@@ -3,6 +3,7 @@
 #include "kfixed.h"
 
 extern "C" const OwlKernelEntry owl_kernel_table_row_a[] = {
+    {"rowx256r4", (const void*)&k_rowx<256, 4, 4, 4, 16>, 64},
     {"rowx256r2", (const void*)&k_rowx<256, 2, 2, 8, 16>, 128},
     {"rowx512r2", (const void*)&k_rowx<512, 2, 2, 16, 16>, 256},
     {"rowx1024r2", (const void*)&k_rowx<1024, 2, 4, 16, 16>, 256},

@@ -320,6 +320,11 @@ template<class E, class F> __device__ __forceinline__ void part(T2& v, int p, F 
     f(v);
   }
 }
+__device__ __forceinline__ void swapIf(bool c, T2& a, T2& b) {
+  const T2 t = a;
+  a = make_double2(c ? b.x : a.x, c ? b.y : a.y);
+  b = make_double2(c ? t.x : b.x, c ? t.y : b.y);
+}
 // v of the lane 8 away in the row of 16 (DPP row rotate by 8)
 __device__ __forceinline__ double lane8(double v) {
   const uint64_t x = __double_as_longlong(v);
@@ -958,6 +963,8 @@ template<int W, int R, int F0, int F1, int F2> struct RowPass {
   __device__ __forceinline__ static int wrapBit(uint64_t meta, int k, int r, int rep) {
     return (int)((uint32_t)(meta >> 32) >> ((k * R + r) * 2 + rep)) & 1;
   }
+  // PIN: line by line in program order (k_rowm, whose registers would spill if lines were interleaved).
+  template<bool PIN = false>
   __device__ __forceinline__ static void carry(const JobDesc& J, const LineW* lwBase, const ColW* cw, uint64_t meta,
                                                T2 (&v)[R][F0], double* cs, double& roe, bool llHere, bool mul3) {
 #pragma unroll
@@ -986,6 +993,10 @@ template<int W, int R, int F0, int F1, int F2> struct RowPass {
           } else {
             v[r][k].x = dgt;
           }
+        }
+        if constexpr (PIN) {
+          pin<1>(&v[r][k]);
+          asm volatile("" : "+v"(cs[k]), "+v"(roe));
         }
       }
     }
@@ -1017,6 +1028,7 @@ template<int W, int R, int F0, int F1, int F2> struct RowPass {
     }
   }
   // Weight, then the forward W-point FFT's stage 0 (radix F0, Ns = 1), in registers.
+  template<bool PIN = false>
   __device__ __forceinline__ static void weightStage0(const LineW* lwBase, const ColW* cw, uint64_t meta, T2 (&v)[R][F0]) {
 #pragma unroll
     for (int r = 0; r < R; ++r) {
@@ -1026,8 +1038,10 @@ template<int W, int R, int F0, int F1, int F2> struct RowPass {
         const double w0 = __builtin_amdgcn_ldexp(lw.w0 * cw[k].w, -wrapBit(meta, k, r, 0));
         const double w1 = __builtin_amdgcn_ldexp(lw.w1 * cw[k].w, -wrapBit(meta, k, r, 1));
         v[r][k] = make_double2(v[r][k].x * w0, v[r][k].y * w1);
+        if constexpr (PIN) { pin<1>(&v[r][k]); }
       }
       Dft<F0, false>::run(v[r]);
+      if constexpr (PIN) { pin<F0>(v[r]); }
     }
   }
   // The other forward stages in LDS. The caller has made sure that no thread still reads the
@@ -1154,6 +1168,253 @@ __global__ __launch_bounds__(W / F0) void k_rowx(const JobDesc* __restrict__ job
   if (mode == ROW_FUSED) { roeGroup(J, roeSlot, roePart, T / 64); }
   P::forwardLds(v, lds, tw, tid, cb);
   P::store(blk, lds, tid);
+}
+
+// ---------------------------------------------------------------- row pass, 16 elements per thread
+// The same pass as k_rowx with fewer LDS trips, for plans with R*F0 = F2 = 16. The first inverse and
+// the last forward stage (radix 16) load and store the block directly: thread (line r, j) holds the
+// frequencies j + k*W/16, and with r fastest in a wave every access is R*16 contiguous bytes of one
+// slot, while the wave that holds j also holds W/16 - j, whose frequencies lie in the other slots of the
+// same lines. Four exchanges go through LDS instead of k_rowx's six trips. SPLIT: real and imaginary parts
+// are exchanged one after the other (half the LDS) in at most 128 VGPRs, at 1024 x 4 four groups and
+// four waves per SIMD on a CU; otherwise complex elements and half the barriers, two waves per SIMD.
+// NT: non-temporal loads and stores; with 4 lines the lanes of j and W/16 - j then trade registers so that one
+// access covers whole 128-byte lines (64-byte halves cost a quarter of the non-temporal bandwidth: 25 against 21 us
+// for the bare copy of 63 MB; with plain accesses they cost nothing).
+// Twiddles: product tables of exact entries in LDS for the middle stages, exact entries of the full
+// table or products of two for the others (Pow16).
+// LDS positions are sums without bank conflicts on the writes: exchanges 1 and 3 (Ns = 1) pad one slot per 16,
+// exchange 4's blocks are F0 slots further apart; the line strides differ so that lanes of R lines at one
+// position do not meet.
+// Measured (HIP events, us per fused launch, k_rowx in parentheses): 1024 x 3840 split 38.5 (43.4), 1024 x 1536 complex
+// 22.5 (24.2), 64 jobs of 256 x 2304 split 277 (340).
+template<int W, int R, int F0, int F1, bool SPLIT> struct RowM {
+  static constexpr int T = W / F0, J = W / 16, F2 = 16, MB = 16 / F1, NB1 = W / F1;
+  static_assert(F0 * F1 * F2 == W && R * F0 == 16 && T % 64 == 0 && NB1 % 16 == 0 && J % 16 == 0, "plan");
+  static constexpr RowLayout G = rowLayout(W, R, F0, F1, SPLIT);
+  static constexpr int L1 = G.l1, L2 = W, L3 = G.l3, L4 = G.l4;  // line strides of the exchanges, in elements
+  static constexpr int KS = G.ks, TAB = G.tab, SLOTS = G.slots;
+  // thread's line and butterfly in the first and last stage
+  __device__ __forceinline__ static int line(int tid) { return tid % R; }
+  __device__ __forceinline__ static int bfly(int tid) {
+    constexpr int U = 64 / R;
+    const int w = tid >> 6, i = (tid & 63) / R;
+    const int lo = w * (U / 2) + i, hi = w * (U / 2) + i - U / 2;
+    return i < U / 2 ? lo : hi ? J - hi : J / 2;
+  }
+  // byte offset of frequency j + k*J of line r within the block
+  __device__ __forceinline__ static uint32_t slotOf(int j, int k, int r) {
+    const int f = j + k * J;
+    const int s = k < 8 ? 2 * f : (k == 8 && f == W / 2) ? 1 : 2 * (W - f) + 1;
+    return (uint32_t)(s * R + r) * 16;
+  }
+};
+
+template<int W, int R, int F0, int F1, bool SPLIT, bool NT, bool FUSED>
+__global__ __launch_bounds__(W / F0, SPLIT ? 4 : 2) void k_rowm(const JobDesc* __restrict__ jobs, int modeArg, int fi, int wi, int opts,
+                                                    uint32_t roeSlot, uint32_t tag) {
+  using M = RowM<W, R, F0, F1, SPLIT>;
+  using P = RowPass<W, R, F0, F1, 16>;
+  constexpr bool FULL = NT && R == 4;
+  constexpr int T = M::T, J_ = M::J, MB = M::MB, NB1 = M::NB1, LW = R * W;
+  const int mode = FUSED ? ROW_FUSED : modeArg;
+  extern __shared__ T2 lds[];
+  using E = std::conditional_t<SPLIT, double, T2>;
+  E* const buf = reinterpret_cast<E*>(lds);
+  T2* const tab = lds + M::TAB;
+  float* const roePart = reinterpret_cast<float*>(lds + M::SLOTS - 4);
+  const JobDesc& J = jobs[blockIdx.y];
+  const int nb = J.nb;
+  __shared__ int ticketSlot;
+  FusedItem it{(int)blockIdx.x, 0, false, false, false, false};
+  if (mode == ROW_FUSED) { it = fusedItem(J, opts, &ticketSlot); }
+  if (it.none) { return; }
+  const int lb = it.lb;
+  const bool ll = opts & 1, mul3 = opts & 2;
+  int tid = threadIdx.x;
+  T2* blk = J.freq[fi] + (size_t)lb * LW;
+
+  T2 x[16];
+  // Exchange: w(m) and r(m) are the LDS addresses of the thread's butterfly m on either side.
+  auto exchange = [&](auto nw, auto mw, auto w, int ws, auto nr, auto mr, auto r, int rs) {
+#pragma unroll
+    for (int p = 0; p < (SPLIT ? 2 : 1); ++p) {
+      __syncthreads();
+#pragma unroll
+      for (int m = 0; m < mw; ++m) {
+        E* d = buf + w(m);
+#pragma unroll
+        for (int k = 0; k < nw; ++k) { part<E>(x[m * nw + k], p, [&](auto& e) { d[k * ws] = e; }); }
+      }
+      __syncthreads();
+#pragma unroll
+      for (int m = 0; m < mr; ++m) {
+        const E* d = buf + r(m);
+#pragma unroll
+        for (int k = 0; k < nr; ++k) { part<E>(x[m * nr + k], p, [&](auto& e) { e = d[k * rs]; }); }
+      }
+    }
+  };
+  constexpr std::integral_constant<int, 1> c1;
+  constexpr std::integral_constant<int, 16> c16;
+  constexpr std::integral_constant<int, F0> cF0;
+  constexpr std::integral_constant<int, F1> cF1;
+  constexpr std::integral_constant<int, MB> cMB;
+  constexpr std::integral_constant<int, R> cR;
+  // middle-stage butterfly m of the thread: line and index
+  auto line1 = [&](int m) { return (tid + m * T) / NB1; };
+  auto bfly1 = [&](int m) { return (tid + m * T) % NB1; };
+
+  if (mode == ROW_LEADIN) {
+    fillProd<16, F1 - 1, M::KS>(J.twRow, F0, tab, tid, T);
+    const int2* src = J.words[wi] + (size_t)lb * LW;
+#pragma unroll
+    for (int k = 0; k < F0; ++k) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const int2 d = gld(src + (tid + k * T) * R + r);
+        x[r * F0 + k] = make_double2(d.x, d.y);
+      }
+    }
+  } else {
+    {
+      const int r = M::line(tid), j = M::bfly(tid);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const uint32_t o = M::slotOf(j, k, r), o2 = M::slotOf(j, 15 - k, r);
+        const bool up = FULL && (tid & 32);
+        x[k] = ldo<NT>(blk, up ? o2 : o);
+        x[15 - k] = ldo<NT>(blk, up ? o : o2);
+      }
+      if constexpr (FULL) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) { swapIf(tid & 32, x[k], x[15 - k]); }
+      }
+    }
+    fillProd<16, F1 - 1, M::KS>(J.twRow, F0, tab, tid, T);
+    dftSeq<16, true>(x);
+    pin<16>(x);
+    FRESH(tid);
+    // inverse stage 1: radix F1, Ns = 16
+    exchange(c16, c1, [&](int) { return M::line(tid) * M::L1 + M::bfly(tid) * 17; }, 1, cF1, cMB,
+             [&](int m) { return line1(m) * M::L1 + bfly1(m) + (bfly1(m) >> 4); }, NB1 / 16 * 17);
+#pragma unroll
+    for (int m = 0; m < MB; ++m) {
+      const T2* t = tab + (bfly1(m) & 15) * M::KS - 1;
+#pragma unroll
+      for (int k = 1; k < F1; ++k) {
+        x[m * F1 + k] = cmulc(x[m * F1 + k], t[k]);
+        pin<1>(&x[m * F1 + k]);
+      }
+      dftSeq<F1, true>(x + m * F1);
+      pin<F1>(x + m * F1);
+    }
+    FRESH(tid);
+    // inverse stage 2: radix F0, Ns = T: columns tid + k*T of the R lines
+    exchange(cF1, cMB, [&](int m) { return line1(m) * M::L2 + (bfly1(m) & ~15) * F1 + (bfly1(m) & 15); }, 16, cF0, cR,
+             [&](int m) { return m * M::L2 + tid; }, T);
+    T2 w[F0];
+#pragma unroll
+    for (int k = 1; k < F0; ++k) { w[k] = gld(J.twRow + tid * k); }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+#pragma unroll
+      for (int k = 1; k < F0; ++k) { x[r * F0 + k] = cmulc(x[r * F0 + k], w[k]); }
+      Dft<F0, true>::run(x + r * F0);
+      pin<F0>(x + r * F0);
+    }
+    FRESH(tid);
+  }
+
+  const uint64_t meta = gld(J.rowMeta + (size_t)lb * T + tid);
+  const LineW* lwBase = J.lineW + lb * R;
+  T2 (&v)[R][F0] = reinterpret_cast<T2 (&)[R][F0]>(x);
+  if (mode != ROW_LEADIN) {
+    double roe = 0;
+    double cs[F0];
+    {
+      ColW cw[F0];
+#pragma unroll
+      for (int k = 0; k < F0; ++k) { cw[k].iw = ((const GLOBAL ColW*)(J.colW + tid + k * T))->iw; }
+      P::template carry<true>(J, lwBase, cw, meta, v, cs, roe, ll && lb == 0 && tid == 0, mul3);
+    }
+    if (mode == ROW_CARRYOUT) {
+      roeReport(J, roeSlot, (float)roe);
+      int2* dst = J.words[wi] + (size_t)lb * LW;
+#pragma unroll
+      for (int k = 0; k < F0; ++k) {
+        const int c = tid + k * T;
+        gst(J.carry[0] + (size_t)lb * W + c, (int64_t)cs[k]);
+#pragma unroll
+        for (int r = 0; r < R; ++r) { gst(dst + c * R + r, make_int2((int)v[r][k].x, (int)v[r][k].y)); }
+      }
+      return;
+    }
+    if (!it.redo) { P::publish(J, lb, tid, tag, cs); }
+    if (it.first) {
+      roeReport(J, roeSlot, (float)roe);
+      return;
+    }
+    roeWave(roeSlot, (float)roe, roePart);
+    uint64_t got[F0];
+    P::pollPredecessor(J, it, tid, tag, got);
+    P::ripple(J, meta, v, got);
+  }
+  {
+    FRESH(tid);
+    ColW cw[F0];
+#pragma unroll
+    for (int k = 0; k < F0; ++k) { cw[k].w = ((const GLOBAL ColW*)(J.colW + tid + k * T))->w; }
+    P::template weightStage0<true>(lwBase, cw, meta, v);
+  }
+  pin<16>(x);
+  // forward stage 1: radix F1, Ns = F0
+  exchange(cF0, cR, [&](int m) { return m * M::L3 + tid * F0 + (tid * F0 >> 4); }, 1, cF1, cMB,
+           [&](int m) { return line1(m) * M::L3 + bfly1(m) + (bfly1(m) >> 4); }, NB1 / 16 * 17);
+  if (mode == ROW_FUSED) { roeGroup(J, roeSlot, roePart, T / 64); }
+#pragma unroll
+  for (int m = 0; m < MB; ++m) {
+    const T2* t = tab + (bfly1(m) % F0) * (16 / F0) * M::KS - 1;
+#pragma unroll
+    for (int k = 1; k < F1; ++k) {
+      x[m * F1 + k] = cmul(x[m * F1 + k], t[k]);
+      pin<1>(&x[m * F1 + k]);
+    }
+    dftSeq<F1, false>(x + m * F1);
+    pin<F1>(x + m * F1);
+  }
+  FRESH(tid);
+  // forward stage 2: radix 16, Ns = J, then the store
+  Pow16 wt;
+  {
+    const int j = M::bfly(tid);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      wt.lo[k] = gld(J.twRow + (k + 1) * j);
+      wt.hi[k] = gld(J.twRow + 4 * (k + 1) * j);
+    }
+  }
+  exchange(cF1, cMB, [&](int m) { return line1(m) * M::L4 + bfly1(m) + bfly1(m) / F0 * J_; }, F0, c16, c1,
+           [&](int) { return M::line(tid) * M::L4 + M::bfly(tid); }, J_ + F0);
+#pragma unroll
+  for (int k = 1; k < 16; ++k) {
+    x[k] = cmul(x[k], wt(k));
+    pin<1>(&x[k]);
+  }
+  dftSeq<16, false>(x);
+  pin<16>(x);
+  FRESH(tid);
+  {
+    const int r = M::line(tid), j = M::bfly(tid);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const uint32_t o = M::slotOf(j, k, r), o2 = M::slotOf(j, 15 - k, r);
+      const bool up = FULL && (tid & 32);
+      if constexpr (FULL) { swapIf(tid & 32, x[k], x[15 - k]); }
+      sto<NT>(blk, up ? o2 : o, x[k]);
+      sto<NT>(blk, up ? o : o2, x[15 - k]);
+    }
+  }
 }
 
 // ---------------------------------------------------------------- name tables
