@@ -196,7 +196,7 @@ Gpu::Gpu(u32 E, const FFTConfig& fftIn, const GpuOptions& optIn) : E{E}, fft{fft
   // ---- tables: twiddles shared per shape (TrigBufCache), weights per exponent (long double, rounded once)
   const u32 step = stepOf(N, E);
   const u32 nHi = (H + 63) / 64;
-  trig_ = TrigBufCache::get(W, H, useY, queue_);
+  trig_ = TrigBufCache::get(W, H, useX ? ColKind::Mirrored : useY ? ColKind::OneRegion : ColKind::Generic, queue_);
   std::vector<LineW> lineW(H);
   for (u32 l = 0; l < H; ++l) {
     for (u32 rep = 0; rep < 2; ++rep) {
@@ -241,6 +241,7 @@ Gpu::Gpu(u32 E, const FFTConfig& fftIn, const GpuOptions& optIn) : E{E}, fft{fft
   J.twPair = trig_->pair.get();
   J.twMidS = trig_->midS.get();
   J.twMidM = trig_->midM.get();
+  J.twMidBase = trig_->midBase.get();
   J.colTab = trig_->colTab.get();
   J.lineW = upload(lineW);
   J.colW = upload(colW);

@@ -2,7 +2,7 @@
 
 #include <cmath>
 
-std::pair<double, double> root1(u32 n, u64 k) {
+static std::pair<long double, long double> rootL(u32 n, u64 k) {
   k %= n;
   // 8k = o*n + rem: angle = (pi/4)(o + rem/n), x = (pi/4) rem/n, y = (pi/4) - x.
   u64 K = 8 * k;
@@ -29,7 +29,17 @@ std::pair<double, double> root1(u32 n, u64 k) {
     c = cc[o / 2];
     s = ss[o / 2];
   }
-  return {double(c), double(-s)};
+  return {c, -s};
+}
+
+std::pair<double, double> root1(u32 n, u64 k) {
+  const auto [c, s] = rootL(n, k);
+  return {double(c), double(s)};
+}
+
+std::pair<double, double> root1Low(u32 n, u64 k) {
+  const auto [c, s] = rootL(n, k);
+  return {double(c - (long double)double(c)), double(s - (long double)double(s))};
 }
 
 std::vector<u32> fftPlan(u32 L) {

@@ -16,7 +16,7 @@ std::vector<double2> colTabOf(u32 H) {
   const ColRadices r = colRadices(H);
   if (!r.c0) { return {}; }
   const u32 KS = (r.c1 - 1) | 1, ROOTS = 256;
-  std::vector<double2> t(colTabLds(H) + 6 * ROOTS, double2{0, 0});
+  std::vector<double2> t(colTabLds(H) + 8 * ROOTS, double2{0, 0});
   auto product = [&](u32 at, u32 rows, u32 n) {  // w_n^(p*k), p < rows, 1 <= k < C1
     for (u32 p = 0; p < rows; ++p) {
       for (u32 k = 1; k < u32(r.c1); ++k) { t[at + p * KS + k - 1] = d2(root1(n, p * k)); }
@@ -24,45 +24,64 @@ std::vector<double2> colTabOf(u32 H) {
   };
   product(0, r.c0, r.c0 * r.c1);
   if (r.c2 != r.c0) { product(r.c0 * KS, r.c2, r.c2 * r.c1); }
-  const u32 m[6] = {1, 2, 3, 4, 8, 12};
-  for (u32 i = 0; i < 6; ++i) {
-    for (u32 k = 0; k < ROOTS; ++k) { t[colTabLds(H) + i * ROOTS + k] = d2(root1(H, m[i] * k)); }
+  for (u32 m = 0; m < 8; ++m) {
+    for (u32 k = 0; k < ROOTS; ++k) { t[colTabLds(H) + m * ROOTS + k] = d2(root1(H, (m + 1) * k)); }
   }
   return t;
 }
 }  // namespace
 
-std::shared_ptr<const TrigTables> TrigBufCache::get(u32 W, u32 H, bool oneRegion, owl_queue q) {
+std::shared_ptr<const TrigTables> TrigBufCache::get(u32 W, u32 H, ColKind kind, owl_queue q) {
   static std::mutex mtx;
-  static std::map<std::tuple<u32, u32, bool>, std::weak_ptr<const TrigTables>> cache;
+  static std::map<std::tuple<u32, u32, ColKind>, std::weak_ptr<const TrigTables>> cache;
   std::lock_guard<std::mutex> lock(mtx);
-  auto key = std::make_tuple(W, H, oneRegion);
+  auto key = std::make_tuple(W, H, kind);
   if (auto it = cache.find(key); it != cache.end()) {
     if (auto sp = it->second.lock()) { return sp; }
   }
   const u32 ND = W * H;
-  const u32 nHi = (H + 63) / 64;
-  std::vector<double2> row(W), col(H), midA(size_t(W) * 64), midB(size_t(W) * nHi), pair(W), mid(size_t(W) * 16);
-  for (u32 m = 0; m < W; ++m) { row[m] = d2(root1(W, m)); }
-  for (u32 m = 0; m < H; ++m) { col[m] = d2(root1(H, m)); }
-  for (u32 a = 0; a < W; ++a) {
-    pair[a] = d2(root1(ND, a));
-    for (u32 lo = 0; lo < 64; ++lo) { midA[size_t(a) * 64 + lo] = d2(root1(ND, u64(a) * lo)); }
-    for (u32 hi = 0; hi < nHi; ++hi) { midB[size_t(a) * nHi + hi] = d2(root1(ND, u64(a) * 64 * hi % ND)); }
-  }
   auto t = std::make_shared<TrigTables>();
-  t->row = Buffer<double2>(q, row);
-  t->col = Buffer<double2>(q, col);
-  t->midA = Buffer<double2>(q, midA);
-  t->midB = Buffer<double2>(q, midB);
-  t->pair = Buffer<double2>(q, pair);
-  const u32 c0 = oneRegion ? 16 : colRadices(H).c0;
-  if (c0) {
-    for (u32 a = 0; a < W; ++a) {
-      for (u32 k = 0; k < 16; ++k) { mid[size_t(a) * 16 + k] = d2(root1(ND, u64(a) * k * (H / c0) % ND)); }
+  // n entries exp(-2 pi i f(i) / L)
+  auto table = [&](u32 n, u32 L, auto f) {
+    std::vector<double2> v(n);
+    for (u32 i = 0; i < n; ++i) { v[i] = d2(root1(L, f(i))); }
+    return Buffer<double2>(q, v);
+  };
+  t->row = table(W, W, [](u32 m) { return u64(m); });
+  t->col = table(H, H, [](u32 m) { return u64(m); });
+  t->pair = table(W, ND, [](u32 a) { return u64(a); });
+  if (kind != ColKind::Mirrored) {
+    const u32 nHi = (H + 63) / 64;
+    t->midA = table(W * 64, ND, [](u32 i) { return u64(i / 64) * (i % 64); });
+    t->midB = table(W * nHi, ND, [=](u32 i) { return u64(i / nHi) * 64 * (i % nHi); });
+    if (kind == ColKind::OneRegion) {
+      t->midS = table(W * 16, ND, [=](u32 i) { return u64(i / 16) * (i % 16) * (H / 16); });
     }
-    (oneRegion ? t->midS : t->midM) = Buffer<double2>(q, mid);
-    if (!oneRegion) { t->colTab = Buffer<double2>(q, colTabOf(H)); }
+  } else {
+    const u32 NB0 = H / colRadices(H).c0, rows = W / 2 + 1, nHi = (NB0 + 63) / 64;
+    t->midM = table(W * 16, ND, [=](u32 i) { return u64(i / 16) * (i % 16) * NB0; });
+    t->colTab = Buffer<double2>(q, colTabOf(H));
+    // midBase: products of two factors with their low parts, rounded once, on the device: per row 64 low factors
+    // exp(-2 pi i a*lo / ND) and nHi high ones, each with its low part after it
+    const u32 per = 2 * (64 + nHi);
+    std::vector<double2> f(size_t(rows) * per);
+    for (u32 a = 0; a < rows; ++a) {
+      for (u32 i = 0; i < 64 + nHi; ++i) {
+        const u64 k = i < 64 ? u64(a) * i : u64(a) * 64 * (i - 64);
+        f[size_t(a) * per + 2 * i] = d2(root1(ND, k));
+        f[size_t(a) * per + 2 * i + 1] = d2(root1Low(ND, k));
+      }
+    }
+    Buffer<double2> factors(q, f);
+    t->midBase = Buffer<double2>(size_t(rows) * NB0);
+    owl_kernel k = nullptr;
+    owlCheck(owl_hip_kernel_get("midBase", &k), "kernel");
+    double2* out = t->midBase.get();
+    const double2* in = factors.get();
+    u32 nb0 = NB0, n = rows * NB0, nh = nHi;
+    void* args[] = {&out, &in, &nb0, &nh, &n};
+    owlCheck(owl_hip_launch(q, k, (n + 255) / 256, 1, 256, 0, args), "midBase");
+    owlCheck(owl_hip_finish(q), "midBase");
   }
   cache[key] = t;
   return t;

@@ -61,6 +61,7 @@ struct JobDesc {
   const double2* twPair;  // W entries: exp(-2 pi i a / ND)
   const double2* twMidS;  // W*16: exp(-2 pi i a*k*(H/16) / ND), k < 16 (shape-specialized column pass)
   const double2* twMidM;  // W*16: exp(-2 pi i a*k*(H/C0) / ND), k < 16, C0 the mirrored column pass's first radix (coltab.h)
+  const double2* twMidBase;  // (W/2+1)*(H/C0): exp(-2 pi i a*j / ND), j < H/C0 (mirrored column pass)
   const double2* colTab;  // twiddle table of the mirrored column pass (coltab.h), null where it has none
   const LineW* lineW;     // H entries
   const ColW* colW;       // W entries

@@ -515,6 +515,29 @@ __global__ __launch_bounds__(256) void k_copy_words(const JobDesc* __restrict__ 
   for (uint32_t p = blockIdx.x * 256 + threadIdx.x; p < J.ND; p += gridDim.x * 256) { J.words[dst][p] = J.words[src][p]; }
 }
 
+// Mid twiddles of the mirrored column pass: out[a*NB0 + j] = exp(-2 pi i a*j / ND), the product of the row's low factor
+// j mod 64 and high factor j div 64 (in: per row a the 64 + nHi factors, each followed by its low part) to about
+// 2^-64, rounded once.
+__global__ __launch_bounds__(256) void k_mid_base(double2* out, const double2* in, uint32_t NB0, uint32_t nHi, uint32_t n) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) { return; }
+  const uint32_t a = i / NB0, j = i % NB0;
+  const double2* f = in + (size_t)a * 2 * (64 + nHi);
+  const double2 x = f[2 * (j & 63)], xl = f[2 * (j & 63) + 1], y = f[2 * (64 + (j >> 6))], yl = f[2 * (64 + (j >> 6)) + 1];
+  // p*q + r*s with the rounding errors of both products and of the sum, and the low parts. The products are kept from
+  // being fused into the sum, which would make their error terms wrong (the build contracts across statements).
+  auto dot = [](double p, double q, double r, double s, double low) {
+    double u = p * q, v = r * s;
+    asm volatile("" : "+v"(u), "+v"(v));
+    const double ue = fma(p, q, -u), ve = fma(r, s, -v);
+    const double h = u + v, b = h - u, he = (u - (h - b)) + (v - b);
+    return h + (he + (ue + ve + low));
+  };
+  const double re = dot(x.x, y.x, -x.y, y.y, x.x * yl.x + xl.x * y.x - x.y * yl.y - xl.y * y.y);
+  const double im = dot(x.x, y.y, x.y, y.x, x.x * yl.y + xl.x * y.y + x.y * yl.x + xl.y * y.x);
+  out[i] = make_double2(re, im);
+}
+
 // ---------------------------------------------------------------- kernel table
 // Looked up by name through owl_hip_kernel_get (the replacement of the reference's
 // named kernel loading, src/clwrap.cpp:278-284).
@@ -541,6 +564,7 @@ extern "C" const OwlKernelEntry owl_kernel_table[] = {
     {"isEqual", (const void*)&k_is_equal, 256},
     {"sum64", (const void*)&k_sum64, 256},
     {"fill32", (const void*)&k_fill32, 256},
+    {"midBase", (const void*)&k_mid_base, 256},
     {"copyWords", (const void*)&k_copy_words, 256},
     {nullptr, nullptr, 0},
 };

@@ -334,51 +334,67 @@ __device__ __forceinline__ double lane8(double v) {
 }
 __device__ __forceinline__ T2 lane8(T2 v) { return make_double2(lane8(v.x), lane8(v.y)); }
 
-// w^k for 1 <= k < 16 from the six exact powers w^1, w^2, w^3, w^4, w^8, w^12: at most one product.
-struct Pow16 {
-  T2 lo[3], hi[3];
-  __device__ __forceinline__ T2 operator()(int k) const {
-    if (k % 4 == 0) { return hi[k / 4 - 1]; }
-    if (k < 4) { return lo[k - 1]; }
-    return cmul(hi[k / 4 - 1], lo[k % 4 - 1]);
-  }
+// w^k for 1 <= k < C <= 16 from the exact powers up to w^8: exact, or one product with w^8. (Six powers 1, 2, 3, 4, 8, 12
+// would do with fewer loads, but the larger share of products raised the error of a squaring by 1 to 3%.)
+template<int C> struct Powers {
+  static constexpr int N = C <= 8 ? C - 1 : 8;
+  T2 w[N];
+  __device__ __forceinline__ T2 operator()(int k) const { return k <= 8 ? w[k - 1] : cmul(w[7], w[k - 9]); }
 };
 
 // Dft<R> with the sub-transforms of a composite R kept one after the other: left to itself the
 // scheduler interleaves them, and their temporaries spill.
-template<int R> struct Split {
+template<int R> struct Coprime {
   static constexpr int P = 0, Q = 0;
 };
-template<> struct Split<15> { static constexpr int P = 3, Q = 5; };
-template<> struct Split<14> { static constexpr int P = 2, Q = 7; };
-template<> struct Split<12> { static constexpr int P = 4, Q = 3; };
-template<> struct Split<16> { static constexpr int P = 4, Q = 4; };
+template<> struct Coprime<10> { static constexpr int P = 2, Q = 5; };
+template<> struct Coprime<14> { static constexpr int P = 2, Q = 7; };
+template<> struct Coprime<15> { static constexpr int P = 3, Q = 5; };
 template<int R, bool INV> __device__ __forceinline__ void dftSeq(T2* a) {
-  constexpr int P = Split<R>::P, Q = Split<R>::Q;
+  constexpr int P = Coprime<R>::P, Q = Coprime<R>::Q;
   pin<R>(a);
-  if constexpr (P == 0) {
-    Dft<R, INV>::run(a);
-  } else {
+  if constexpr (P != 0) {
     T2 b[Q][P];
 #pragma unroll
-    for (int k2 = 0; k2 < Q; ++k2) {
+    for (int n2 = 0; n2 < Q; ++n2) {
 #pragma unroll
-      for (int k1 = 0; k1 < P; ++k1) { b[k2][k1] = a[Q * k1 + k2]; }
-      Dft<P, INV>::run(b[k2]);
-#pragma unroll
-      for (int m1 = 1; m1 < P; ++m1) { b[k2][m1] = rootMul<R, INV>(b[k2][m1], k2 * m1); }
-      pin<P>(b[k2]);
+      for (int n1 = 0; n1 < P; ++n1) { b[n2][n1] = a[pfaIn<P, Q>(n1, n2)]; }
+      Dft<P, INV>::run(b[n2]);
+      pin<P>(b[n2]);
     }
 #pragma unroll
-    for (int m1 = 0; m1 < P; ++m1) {
+    for (int k1 = 0; k1 < P; ++k1) {
       T2 c[Q];
 #pragma unroll
-      for (int k2 = 0; k2 < Q; ++k2) { c[k2] = b[k2][m1]; }
+      for (int n2 = 0; n2 < Q; ++n2) { c[n2] = b[n2][k1]; }
       Dft<Q, INV>::run(c);
       pin<Q>(c);
 #pragma unroll
-      for (int m2 = 0; m2 < Q; ++m2) { a[m1 + P * m2] = c[m2]; }
+      for (int k2 = 0; k2 < Q; ++k2) { a[pfaOut<P, Q>(k1, k2)] = c[k2]; }
     }
+  } else if constexpr (R == 16) {
+    T2 b[4][4];
+#pragma unroll
+    for (int k2 = 0; k2 < 4; ++k2) {
+#pragma unroll
+      for (int k1 = 0; k1 < 4; ++k1) { b[k2][k1] = a[4 * k1 + k2]; }
+      Dft<4, INV>::run(b[k2]);
+#pragma unroll
+      for (int m1 = 1; m1 < 4; ++m1) { b[k2][m1] = rootMul<16, INV>(b[k2][m1], k2 * m1); }
+      pin<4>(b[k2]);
+    }
+#pragma unroll
+    for (int m1 = 0; m1 < 4; ++m1) {
+      T2 c[4];
+#pragma unroll
+      for (int k2 = 0; k2 < 4; ++k2) { c[k2] = b[k2][m1]; }
+      Dft<4, INV>::run(c);
+      pin<4>(c);
+#pragma unroll
+      for (int m2 = 0; m2 < 4; ++m2) { a[m1 + 4 * m2] = c[m2]; }
+    }
+  } else {
+    Dft<R, INV>::run(a);
   }
 }
 
@@ -420,7 +436,7 @@ __global__ __launch_bounds__(T, SPLIT ? 4 : 2) void k_colx(const JobDesc* __rest
   // its own; the latter pairs with itself, so it is not conjugated.
   const int a = q ? q : W / 2;
   const double sgn = (q && h) ? -1.0 : 1.0;
-  auto midBase = [&](int l) -> T2 { return cmul(gld(J.twMidA + a * 64 + (l & 63)), gld(J.twMidB + a * J.nHi + (l >> 6))); };
+  auto midBase = [&](int l) -> T2 { return gld(J.twMidBase + a * NB0 + l); };
   auto mid = [&](T2 base, int k) -> T2 {
     const CONSTANT double* s = (const CONSTANT double*)(J.twMidM + a * 16 + k);
     T2 w = k ? cmul(base, make_double2(s[0], s[1])) : base;
@@ -430,13 +446,10 @@ __global__ __launch_bounds__(T, SPLIT ? 4 : 2) void k_colx(const JobDesc* __rest
     }
     return w;
   };
-  auto loadWt = [&](Pow16& wt, int t0) {  // w_H^(j*k)
+  auto loadWt = [&](auto& wt, int t0) {  // w_H^(j*k)
     const T2* t = J.colTab + L::LDS + t0;
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      wt.lo[k] = gld(t + k * L::ROOTS);
-      wt.hi[k] = gld(t + (3 + k) * L::ROOTS);
-    }
+    for (int k = 0; k < wt.N; ++k) { wt.w[k] = gld(t + k * L::ROOTS); }
   };
 
   constexpr std::integral_constant<int, C0> c0;
@@ -499,13 +512,13 @@ __global__ __launch_bounds__(T, SPLIT ? 4 : 2) void k_colx(const JobDesc* __rest
   }
   FRESH(j);
   // stage 2: radix C2, Ns = C0*C1 = NB2: bins j + k*NB2
-  Pow16 wt;
+  Powers<C2> wt;
   loadWt(wt, jP);
   {  // blocks of C0*C1 = NB2 elements, C0 further apart
     const int j1 = bf(NB1), blk = j1 / C0;
     exchange(c1, NB1, reg + j1 + blk * NB2, C0, c2, NB2, regP + jP, NB2 + C0);
   }
-  T2 wb = wt.lo[0];
+  T2 wb = wt.w[0];
 #pragma unroll
   for (int k = 1; k < C2; ++k) {
     x[k] = cmul(x[k], wt(k));
@@ -603,7 +616,8 @@ __global__ __launch_bounds__(T, SPLIT ? 4 : 2) void k_colx(const JobDesc* __rest
   FRESH(j);
   // stage 2: radix C0, Ns = NB0, then the conjugate mid twiddle and the store
   const int j0 = bf(NB0);
-  loadWt(wt, j0);
+  Powers<C0> wi;
+  loadWt(wi, j0);
   {  // blocks of C1*C2 = NB0 elements, C2 further apart
     const int j1 = bf(NB1), blk = j1 / C2;
     exchange(c1, NB1, reg + j1 + blk * NB0, C2, c0, NB0, reg + j0, NB0 + C2);
@@ -611,7 +625,7 @@ __global__ __launch_bounds__(T, SPLIT ? 4 : 2) void k_colx(const JobDesc* __rest
   if (runs(NB0)) {
 #pragma unroll
     for (int k = 1; k < C0; ++k) {
-      x[k] = cmulc(x[k], wt(k));
+      x[k] = cmulc(x[k], wi(k));
       pin<1>(&x[k]);
     }
     dftSeq<C0, true>(x);
@@ -1182,7 +1196,7 @@ __global__ __launch_bounds__(W / F0) void k_rowx(const JobDesc* __restrict__ job
 // access covers whole 128-byte lines (64-byte halves cost a quarter of the non-temporal bandwidth: 25 against 21 us
 // for the bare copy of 63 MB; with plain accesses they cost nothing).
 // Twiddles: product tables of exact entries in LDS for the middle stages, exact entries of the full
-// table or products of two for the others (Pow16).
+// table or products of two for the others (Powers).
 // LDS positions are sums without bank conflicts on the writes: exchanges 1 and 3 (Ns = 1) pad one slot per 16,
 // exchange 4's blocks are F0 slots further apart; the line strides differ so that lanes of R lines at one
 // position do not meet.
@@ -1385,14 +1399,11 @@ __global__ __launch_bounds__(W / F0, SPLIT ? 4 : 2) void k_rowm(const JobDesc* _
   }
   FRESH(tid);
   // forward stage 2: radix 16, Ns = J, then the store
-  Pow16 wt;
+  Powers<16> wt;
   {
     const int j = M::bfly(tid);
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      wt.lo[k] = gld(J.twRow + (k + 1) * j);
-      wt.hi[k] = gld(J.twRow + 4 * (k + 1) * j);
-    }
+    for (int k = 0; k < 8; ++k) { wt.w[k] = gld(J.twRow + (k + 1) * j); }
   }
   exchange(cF1, cMB, [&](int m) { return line1(m) * M::L4 + bfly1(m) + bfly1(m) / F0 * J_; }, F0, c16, c1,
            [&](int) { return M::line(tid) * M::L4 + M::bfly(tid); }, J_ + F0);
