@@ -16,7 +16,7 @@ std::vector<double2> colTabOf(u32 H) {
   const ColRadices r = colRadices(H);
   if (!r.c0) { return {}; }
   const u32 KS = (r.c1 - 1) | 1, ROOTS = 256;
-  std::vector<double2> t(colTabLds(H) + 8 * ROOTS, double2{0, 0});
+  std::vector<double2> t(colTabLds(H) + 15 * ROOTS, double2{0, 0});
   auto product = [&](u32 at, u32 rows, u32 n) {  // w_n^(p*k), p < rows, 1 <= k < C1
     for (u32 p = 0; p < rows; ++p) {
       for (u32 k = 1; k < u32(r.c1); ++k) { t[at + p * KS + k - 1] = d2(root1(n, p * k)); }
@@ -24,7 +24,7 @@ std::vector<double2> colTabOf(u32 H) {
   };
   product(0, r.c0, r.c0 * r.c1);
   if (r.c2 != r.c0) { product(r.c0 * KS, r.c2, r.c2 * r.c1); }
-  for (u32 m = 0; m < 8; ++m) {
+  for (u32 m = 0; m < 15; ++m) {
     for (u32 k = 0; k < ROOTS; ++k) { t[colTabLds(H) + m * ROOTS + k] = d2(root1(H, (m + 1) * k)); }
   }
   return t;

@@ -6,7 +6,7 @@
 // product tables with rows of odd stride KS,
 //   A: w_(C0*C1)^(p*k), p < C0, 1 <= k < C1, at p*KS + k - 1 (forward stage 1)
 //   B: w_(C2*C1)^(p*k), p < C2 (inverse stage 1); A itself when C2 = C0
-// then eight rows of ROOTS entries, w_H^(m*t) for m = 1 ... 8 and t < ROOTS, which thread t reads.
+// then 15 rows of ROOTS entries, w_H^(m*t) for m = 1 ... 15 and t < ROOTS, which thread t reads.
 template<int H, int C0, int C1, int C2> struct ColTab {
   static constexpr int KS = (C1 - 1) | 1;
   static constexpr int A = 0;

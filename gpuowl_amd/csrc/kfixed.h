@@ -334,12 +334,25 @@ __device__ __forceinline__ double lane8(double v) {
 }
 __device__ __forceinline__ T2 lane8(T2 v) { return make_double2(lane8(v.x), lane8(v.y)); }
 
-// w^k for 1 <= k < C <= 16 from the exact powers up to w^8: exact, or one product with w^8. (Six powers 1, 2, 3, 4, 8, 12
-// would do with fewer loads, but the larger share of products raised the error of a squaring by 1 to 3%.)
+// x[k] *= w^k (conj: by its conjugate) for 1 <= k < C <= 16, w^k exact from load(k): the first six loaded beforehand
+// (w), each later one into the registers of the one six before it, which is used up. (Products of loaded powers raised the
+// error of a squaring by 1 to 3%.)
 template<int C> struct Powers {
-  static constexpr int N = C <= 8 ? C - 1 : 8;
+  static constexpr int N = C <= 6 ? C - 1 : 6;
   T2 w[N];
-  __device__ __forceinline__ T2 operator()(int k) const { return k <= 8 ? w[k - 1] : cmul(w[7], w[k - 9]); }
+  template<typename Load> __device__ __forceinline__ void begin(Load load) {
+#pragma unroll
+    for (int k = 1; k <= N; ++k) { w[k - 1] = load(k); }
+  }
+  template<bool CONJ, typename Load> __device__ __forceinline__ void apply(T2* x, Load load) {
+#pragma unroll
+    for (int k = 1; k < C; ++k) {
+      T2& t = w[(k - 1) % N];
+      x[k] = CONJ ? cmulc(x[k], t) : cmul(x[k], t);
+      pin<1>(&x[k]);
+      if (k + N < C) { t = load(k + N); }
+    }
+  }
 };
 
 // Dft<R> with the sub-transforms of a composite R kept one after the other: left to itself the
@@ -446,11 +459,7 @@ __global__ __launch_bounds__(T, SPLIT ? 4 : 2) void k_colx(const JobDesc* __rest
     }
     return w;
   };
-  auto loadWt = [&](auto& wt, int t0) {  // w_H^(j*k)
-    const T2* t = J.colTab + L::LDS + t0;
-#pragma unroll
-    for (int k = 0; k < wt.N; ++k) { wt.w[k] = gld(t + k * L::ROOTS); }
-  };
+  auto root = [&](int t, int k) -> T2 { return gld(J.colTab + L::LDS + t + (k - 1) * L::ROOTS); };  // w_H^(t*k)
 
   constexpr std::integral_constant<int, C0> c0;
   constexpr std::integral_constant<int, C1> c1;
@@ -513,17 +522,13 @@ __global__ __launch_bounds__(T, SPLIT ? 4 : 2) void k_colx(const JobDesc* __rest
   FRESH(j);
   // stage 2: radix C2, Ns = C0*C1 = NB2: bins j + k*NB2
   Powers<C2> wt;
-  loadWt(wt, jP);
+  wt.begin([&](int k) { return root(jP, k); });
   {  // blocks of C0*C1 = NB2 elements, C0 further apart
     const int j1 = bf(NB1), blk = j1 / C0;
     exchange(c1, NB1, reg + j1 + blk * NB2, C0, c2, NB2, regP + jP, NB2 + C0);
   }
   T2 wb = wt.w[0];
-#pragma unroll
-  for (int k = 1; k < C2; ++k) {
-    x[k] = cmul(x[k], wt(k));
-    pin<1>(&x[k]);
-  }
+  wt.template apply<false>(x, [&](int k) { return root(jP, k); });
   dftSeq<C2, false>(x);
   pin<C2>(x);
   FRESH(jP);
@@ -617,17 +622,13 @@ __global__ __launch_bounds__(T, SPLIT ? 4 : 2) void k_colx(const JobDesc* __rest
   // stage 2: radix C0, Ns = NB0, then the conjugate mid twiddle and the store
   const int j0 = bf(NB0);
   Powers<C0> wi;
-  loadWt(wi, j0);
+  wi.begin([&](int k) { return root(j0, k); });
   {  // blocks of C1*C2 = NB0 elements, C2 further apart
     const int j1 = bf(NB1), blk = j1 / C2;
     exchange(c1, NB1, reg + j1 + blk * NB0, C2, c0, NB0, reg + j0, NB0 + C2);
   }
   if (runs(NB0)) {
-#pragma unroll
-    for (int k = 1; k < C0; ++k) {
-      x[k] = cmulc(x[k], wi(k));
-      pin<1>(&x[k]);
-    }
+    wi.template apply<true>(x, [&](int k) { return root(j0, k); });
     dftSeq<C0, true>(x);
     pin<C0>(x);
     FRESH(j);
@@ -1052,7 +1053,6 @@ template<int W, int R, int F0, int F1, int F2> struct RowPass {
         const double w0 = __builtin_amdgcn_ldexp(lw.w0 * cw[k].w, -wrapBit(meta, k, r, 0));
         const double w1 = __builtin_amdgcn_ldexp(lw.w1 * cw[k].w, -wrapBit(meta, k, r, 1));
         v[r][k] = make_double2(v[r][k].x * w0, v[r][k].y * w1);
-        if constexpr (PIN) { pin<1>(&v[r][k]); }
       }
       Dft<F0, false>::run(v[r]);
       if constexpr (PIN) { pin<F0>(v[r]); }
@@ -1196,7 +1196,7 @@ __global__ __launch_bounds__(W / F0) void k_rowx(const JobDesc* __restrict__ job
 // access covers whole 128-byte lines (64-byte halves cost a quarter of the non-temporal bandwidth: 25 against 21 us
 // for the bare copy of 63 MB; with plain accesses they cost nothing).
 // Twiddles: product tables of exact entries in LDS for the middle stages, exact entries of the full
-// table or products of two for the others (Powers).
+// table for the others (Powers).
 // LDS positions are sums without bank conflicts on the writes: exchanges 1 and 3 (Ns = 1) pad one slot per 16,
 // exchange 4's blocks are F0 slots further apart; the line strides differ so that lanes of R lines at one
 // position do not meet.
@@ -1400,18 +1400,10 @@ __global__ __launch_bounds__(W / F0, SPLIT ? 4 : 2) void k_rowm(const JobDesc* _
   FRESH(tid);
   // forward stage 2: radix 16, Ns = J, then the store
   Powers<16> wt;
-  {
-    const int j = M::bfly(tid);
-#pragma unroll
-    for (int k = 0; k < 8; ++k) { wt.w[k] = gld(J.twRow + (k + 1) * j); }
-  }
+  wt.begin([&](int k) { return gld(J.twRow + k * M::bfly(tid)); });
   exchange(cF1, cMB, [&](int m) { return line1(m) * M::L4 + bfly1(m) + bfly1(m) / F0 * J_; }, F0, c16, c1,
            [&](int) { return M::line(tid) * M::L4 + M::bfly(tid); }, J_ + F0);
-#pragma unroll
-  for (int k = 1; k < 16; ++k) {
-    x[k] = cmul(x[k], wt(k));
-    pin<1>(&x[k]);
-  }
+  wt.template apply<false>(x, [&](int k) { return gld(J.twRow + k * M::bfly(tid)); });
   dftSeq<16, false>(x);
   pin<16>(x);
   FRESH(tid);
