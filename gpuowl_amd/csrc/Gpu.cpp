@@ -21,6 +21,19 @@ u32 pow2AtLeast(u32 x, u32 lo, u32 hi) {
   return t;
 }
 
+// Width of the W x H split of ND points for a job that runs alone, 0 where the rule has none: the smallest of 256, 512
+// and 1024 with a column pass of at most 2048 lines, and 1024 up to its 4096. Fewer columns than 512 leave
+// compute units without a column pair; more lines per column only lengthen every group's chain of stages.
+// Measured, us per squaring (2-line blocks): ND = 589,824: 256 x 2304 30.1, 512 x 1152 27.2; 851,968: 256 x 3328 41.0 (36.6
+// with 8 lines), 512 x 1664 29.9; 458,752: 256 x 1792 25.8; 1,179,648: 512 x 2304 38.7, 1024 x 1152 34.3.
+u32 aloneWidth(u32 ND) {
+  for (u32 w = 256; w <= 1024; w *= 2) {
+    const u32 h = ND / w;
+    if (ND % w == 0 && h <= (w == 1024 ? 4096u : 2048u) && colRadices(int(h)).c0) { return w; }
+  }
+  return 0;
+}
+
 // Compute units of a device, asked for once.
 u32 computeUnits(int device) {
   static std::mutex mtx;
@@ -80,9 +93,17 @@ Gpu::Gpu(u32 E, const FFTConfig& fftIn, const GpuOptions& optIn) : E{E}, fft{fft
     opt.colOnePair = tuned.colOnePair;
     tunedLineBlock_ = true;
   }
+  // A job that runs alone takes the split and line block that fill the device, whatever the reference's. In the last 0.3%
+  // below the largest exponent of its FFT it keeps the reference's, whose round-off is smaller by up to 11% (a 512 x 2048
+  // split of 2^21 words against 256 x 4096 in 8-line blocks: mean largest error 0.213 against 0.203 at the limit, and
+  // 0.194 at 0.3% below it).
+  const bool alone = !opt.shared && !opt.lineBlock && !opt.generic && !opt.colOneRegion && E <= 0.997 * fft.maxExp();
   if (opt.width) {
     if (ND % opt.width) { throw std::invalid_argument("width does not divide the FFT length"); }
     W = opt.width;
+    H = ND / W;
+  } else if (alone && aloneWidth(ND)) {
+    W = aloneWidth(ND);
     H = ND / W;
   } else if (H > 4096) {
     // The column pass holds a column pair in LDS (H <= 4096). Taller reference shapes
@@ -111,6 +132,11 @@ Gpu::Gpu(u32 E, const FFTConfig& fftIn, const GpuOptions& optIn) : E{E}, fft{fft
     return owl_hip_kernel_get(name.c_str(), &k) == 0;
   };
   R = opt.lineBlock;
+  // a job alone below 3M words: two lines, for more groups with fewer words each (us per squaring: 2,621,440 words 34.9,
+  // 37.5 with four lines; 3,145,728 words 41.0, 38.6 with four)
+  if (!R && alone && N < 3u << 20 && H % 2 == 0 && fusedStable(2) && haveKernel("rowx" + std::to_string(W) + "r2")) {
+    R = 2;
+  }
   if (R && tunedLineBlock_ && (!fusedStable(R) || H % R || R * W > 4096)) { R = 0; }  // tuned for another exponent
   if (!R && !opt.generic) {
     // the largest line block with a shape-specialized row pass that keeps >= 128 groups

@@ -46,7 +46,8 @@ struct GpuOptions {
   bool generic = false;    // runtime-plan kernels even where a shape-specialized pass exists
   bool colOneRegion = false;  // the one-region column pass (k_coly) where k_colx exists
   bool colOnePair = false;    // k_colx without split exchanges, one column pair on a CU at a time
-  u32 width = 0;           // W of the W x H split of the FFT; 0 = the reference's (refactored when too tall)
+  bool shared = false;     // the job's launches are shared by a batch: the reference's split and long line blocks
+  u32 width = 0;           // W of the W x H split of the FFT; 0 = automatic
   u32 lineBlock = 0;       // lines per row-pass block; 0 = automatic
   int device = 0;
 };

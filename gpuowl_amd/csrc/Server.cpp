@@ -92,7 +92,9 @@ void Server::admit() {
     job->res.tSubmit = r.tSubmit;
     job->res.tAdmit = now();
     try {
-      job->gpu = std::make_unique<Gpu>(r.E, fft, opt_.gpu);
+      GpuOptions o = opt_.gpu;
+      o.shared = true;
+      job->gpu = std::make_unique<Gpu>(r.E, fft, o);
     } catch (const std::invalid_argument&) {
       job->res.status = 2;  // rejected: no engine for this exponent
       job->res.tDone = now();
