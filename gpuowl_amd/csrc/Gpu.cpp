@@ -353,6 +353,9 @@ Gpu::Gpu(u32 E, const FFTConfig& fftIn, const GpuOptions& optIn) : E{E}, fft{fft
   kResidue = Kernel("readResidue");
   kIsEqual = Kernel("isEqual");
   kSum64 = Kernel("sum64");
+  kPack = Kernel("pack");
+  kUnpack = Kernel("unpack");
+  keepPacked_ = !opt.shared;
   kCopy = Kernel("copyWords");
   finish();
 }
@@ -596,7 +599,30 @@ void Gpu::writeDigits(Buf b, const std::vector<int>& digits) {
   finish();
 }
 
-void Gpu::writeIn(Buf b, const Words& words) { writeDigits(b, expandBits(words, N, E)); }
+// Device memory for a residue's words behind a PackHead: kept by a job that runs alone, `own` for one of many (which
+// would each hold 2.5 bytes per digit for the rare read or write).
+u32* Gpu::packed(Buffer<u32>& own) {
+  Buffer<u32>& p = keepPacked_ ? packed_ : own;
+  if (!p.get()) { p = Buffer<u32>(sizeof(PackHead) / 4 + nWords(E)); }
+  return p.get();
+}
+
+void Gpu::writeIn(Buf b, const u32* words, size_t n) {
+  if (n == nWords(E)) {
+    Buffer<u32> own;
+    u32* dev = packed(own);
+    u32* data = dev + sizeof(PackHead) / 4;
+    const JobDesc* j = jobs_.get();
+    int wi = b;
+    PackHead head;
+    owlCheck(owl_hip_fill32(queue_, dev, 0, sizeof(head) / 4), "fill");
+    owlCheck(owl_hip_write(queue_, data, words, n * 4, 0), "write");
+    kUnpack(queue_, (ND + 255) / 256, 1, 256, 0, {&j, &wi, &dev, &data});
+    owlCheck(owl_hip_read(queue_, &head, dev, sizeof(head), 1), "read");
+    if (!head.undecided) { return; }
+  }
+  writeDigits(b, expandBits(Words(words, words + n), N, E));
+}
 
 std::vector<int> Gpu::readDigits(Buf b) {
   Buffer<int32_t> seq(N);
@@ -634,12 +660,37 @@ void Gpu::readDigitsVia(Buf b, int32_t* staging, int32_t* out) {
   throw GpuError("persistent GPU read errors");
 }
 
+bool Gpu::readWords(Buf b, u32* out) {
+  Buffer<u32> own;
+  u32* dev = packed(own);
+  u32* data = dev + sizeof(PackHead) / 4;
+  const u32 n = nWords(E);
+  const JobDesc* j = jobs_.get();
+  int wi = b;
+  for (int attempt = 0; attempt < 3; ++attempt) {
+    PackHead head;
+    owlCheck(owl_hip_fill32(queue_, dev, 0, sizeof(head) / 4), "fill");
+    kPack(queue_, std::min((n + 255) / 256, 1024u), 1, 256, 0, {&j, &wi, &dev, &data});
+    owlCheck(owl_hip_read(queue_, &head, dev, sizeof(head), 1), "read");
+    if (head.timedOut) { throw GpuError("carry hand-off timed out"); }
+    if (!head.nonZero) { return false; }
+    if (head.undecided) {
+      const Words w = compactBits(readDigits(b), E);
+      std::copy(w.begin(), w.end(), out);
+      return true;
+    }
+    owlCheck(owl_hip_read(queue_, out, data, size_t(n) * 4, 1), "read");
+    u64 sum = 0;
+    for (u32 i = 0; i < n; ++i) { sum += out[i]; }
+    if (sum == head.sum) { return true; }
+  }
+  throw GpuError("persistent GPU read errors");
+}
+
 Words Gpu::readData(Buf b) {
-  u32 f = flagsRead();
-  if (f & 4) { throw GpuError("carry hand-off timed out"); }
-  std::vector<int> d = readDigits(b);
-  if (std::all_of(d.begin(), d.end(), [](int x) { return x == 0; })) { return {}; }
-  return compactBits(d, E);
+  Words w(nWords(E));
+  if (!readWords(b, w.data())) { return {}; }
+  return w;
 }
 
 u64 Gpu::dataResidue(Buf b) {

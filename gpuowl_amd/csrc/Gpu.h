@@ -97,13 +97,15 @@ public:
   std::vector<u32> rowPlan, colPlan;
 
   // state I/O (src/Gpu.cpp:801-811, 677-705)
-  void writeIn(Buf b, const Words& words);
+  void writeIn(Buf b, const Words& words) { writeIn(b, words.data(), words.size()); }
+  void writeIn(Buf b, const u32* words, size_t n);
   void writeDigits(Buf b, const std::vector<int>& digits);  // sequential balanced digits
   std::vector<int> readDigits(Buf b);                       // sequential digits, checksum-verified
   // readDigits into out (N int32, host) through the library's static staging array instead of
   // a staging buffer allocated per call; rejects N > OWL_NOALLOC_MAX_WORDS
   void readDigitsNoAlloc(Buf b, int32_t* out);
-  Words readData(Buf b = DATA);                             // canonical residue words
+  Words readData(Buf b = DATA);                             // canonical residue words, empty for zero
+  bool readWords(Buf b, u32* out);                          // the same into nWords(E) words; false (out as it was) for zero
   u64 dataResidue(Buf b = DATA);                            // res64 via readResidue (src/Gpu.cpp:955-975)
 
   // the squaring path (src/Gpu.cpp:851-945)
@@ -236,11 +238,14 @@ private:
   bool colX_ = false;   // the column pass is k_colx
   u32 cus_ = 1;         // compute units
   Kernel kRowF[2][2], kColSq[2][2];  // [split][streamed]: fused row pass (rowM), squaring column pass (colX_)
-  Kernel kRow, kCol, kCarryB, kCarryFix, kWordsIn, kWordsOut, kResidue, kIsEqual, kSum64, kCopy;
+  Kernel kRow, kCol, kCarryB, kCarryFix, kWordsIn, kWordsOut, kResidue, kIsEqual, kSum64, kCopy, kPack, kUnpack;
+  Buffer<u32> packed_;       // PackHead and a residue's words, kept by a job that runs alone
+  bool keepPacked_ = false;
 
   template<typename T> T* alloc(size_t n);
   template<typename T> T* upload(const std::vector<T>& v);
   void readDigitsVia(Buf b, int32_t* staging, int32_t* out);
+  u32* packed(Buffer<u32>& own);
 };
 
 // Mersenne-prime type-1 PRP residue is 9 (src/Gpu.cpp:1036-1040).

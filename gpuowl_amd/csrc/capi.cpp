@@ -163,16 +163,16 @@ void fillInfo(const Gpu& G, owl_gpu_info_t* info) {
 }
 
 int owl_gpu_write_words(owl_gpu g, int b, const uint32_t* words, uint32_t n) {
-  return guarded([&] { g->gpu->writeIn(buf(b), Words(words, words + n)); });
+  return guarded([&] { g->gpu->writeIn(buf(b), words, n); });
 }
 
 int owl_gpu_read_words(owl_gpu g, int b, uint32_t* words, uint32_t n, int* isZero) {
   return guarded([&] {
-    Words w = g->gpu->readData(buf(b));
-    *isZero = w.empty();
-    if (!w.empty()) {
-      if (w.size() != n) { throw std::invalid_argument("word count mismatch"); }
-      memcpy(words, w.data(), n * 4);
+    if (n != nWords(g->gpu->E)) {  // refused, unless the residue is zero
+      *isZero = g->gpu->readData(buf(b)).empty();
+      if (!*isZero) { throw std::invalid_argument("word count mismatch"); }
+    } else {
+      *isZero = !g->gpu->readWords(buf(b), words);
     }
   });
 }

@@ -473,6 +473,124 @@ __global__ __launch_bounds__(256) void k_words_out(const JobDesc* __restrict__ j
   seq[2 * j + 1] = v.y;
 }
 
+// ---------------------------------------------------------------- residue words <-> digits
+// A residue's E bits in 32-bit words, low first, from and to the balanced digits of a words buffer (the order of
+// k_words_in). head[] (PackHead, zeroed before): what the host needs to know about the result. One thread per word
+// or pair of digits; a borrow or carry comes from the nearest lower digit that decides it, nearly always the first one
+// looked at. After LOOK digits that do not (a short residue's zeros), or for a digit that no normalized state
+// holds, the kernel sets `undecided` and the host converts the digits itself.
+// Bound by the copy over the host link: at 139M bits 17 MB, and 31 MB of digits in device memory, whose R-line pieces
+// of 8R bytes a thread's neighbours W*R apart complete in the caches. The host took 31 MB each way and a serial loop
+// over the digits; a residue of 139M bits written and read back 37.5 -> 2.6 ms, at 9.5M bits one power step with three
+// residues moved 6.2 -> 3.2 ms.
+constexpr int LOOK = 16;
+
+struct Digits {  // positions and lengths of an exponent's digits
+  uint32_t E, N, lo, rest;
+  __device__ explicit Digits(const JobDesc& J) : E{J.E}, N{J.N}, lo{J.E / J.N}, rest{J.E % J.N} {}
+  __device__ uint64_t pos(uint32_t k) const { return ((uint64_t)k * E + N - 1) / N; }  // first bit of digit k
+  __device__ uint32_t rem(uint32_t k) const { return (uint32_t)(pos(k) * N - (uint64_t)k * E); }
+  // length of the digit whose rem is r, and the next digit's rem
+  __device__ uint32_t len(uint32_t& r) const {
+    const bool big = r < rest;
+    r = big ? r - rest + N : r - rest;
+    return lo + big;
+  }
+};
+
+__device__ __forceinline__ size_t digitAt(const JobDesc& J, uint32_t k) {
+  const uint32_t j = k >> 1, l = j % J.H, c = j / J.H;
+  return 2 * ((size_t)(l / J.R) * J.W * J.R + (size_t)c * J.R + l % J.R) + (k & 1);
+}
+
+__global__ __launch_bounds__(256) void k_pack(const JobDesc* __restrict__ jobs, int wi, PackHead* head, uint32_t* out) {
+  const JobDesc& J = jobs[0];
+  const int32_t* w = (const int32_t*)J.words[wi];
+  const Digits D(J);
+  const uint32_t n = (J.E - 1) / 32 + 1, N = J.N;
+  uint64_t sum = 0;
+  bool undecided = false, nonZero = false;
+  for (uint32_t p = blockIdx.x * 256 + threadIdx.x; p < n; p += gridDim.x * 256) {
+    const uint64_t bit = 32 * (uint64_t)p;
+    uint32_t k = (uint32_t)(bit * N / J.E), r = D.rem(k);
+    int64_t borrow = 0;
+    {
+      uint32_t i = k;
+      int m = 0, d = 0;
+      while (d == 0 && m++ < LOOK) {
+        i = i ? i - 1 : N - 1;
+        d = w[digitAt(J, i)];
+      }
+      undecided |= d == 0;
+      borrow = d < 0 ? -1 : 0;
+    }
+    uint64_t acc = 0;
+    uint32_t have = 0, skip = (uint32_t)(bit - D.pos(k));
+    for (; have < 32 && k < N; ++k) {
+      const uint32_t b = D.len(r);
+      const int d = w[digitAt(J, k)];
+      int64_t v = d + borrow;
+      nonZero |= d != 0;
+      undecided |= d >= (int64_t)1 << b || d <= -((int64_t)1 << b);
+      borrow = 0;
+      if (v < 0) {
+        v += (int64_t)1 << b;
+        borrow = -1;
+      }
+      acc |= ((uint64_t)v >> skip) << have;
+      have += b - skip;
+      skip = 0;
+    }
+    out[p] = (uint32_t)acc;
+    sum += (uint32_t)acc;
+  }
+  for (int off = 32; off > 0; off >>= 1) { sum += __shfl_xor(sum, off, 64); }
+  const bool anyU = __any(undecided), anyN = __any(nonZero);
+  if ((threadIdx.x & 63) == 0) {
+    atomicAdd((unsigned long long*)&head->sum, (unsigned long long)sum);
+    if (anyU) { atomicOr(&head->undecided, 1u); }
+    if (anyN) { atomicOr(&head->nonZero, 1u); }
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) { head->timedOut = J.flags[2]; }
+}
+
+__global__ __launch_bounds__(256) void k_unpack(const JobDesc* __restrict__ jobs, int wi, PackHead* head, const uint32_t* in) {
+  const JobDesc& J = jobs[0];
+  const Digits D(J);
+  const uint32_t n = (J.E - 1) / 32 + 1, N = J.N, j = blockIdx.x * 256 + threadIdx.x;
+  if (j >= J.ND) { return; }
+  auto raw = [&](uint32_t k, uint32_t& b) -> uint64_t {
+    uint32_t r = D.rem(k);
+    const uint64_t at = D.pos(k);
+    const uint32_t i = (uint32_t)(at >> 5);
+    b = D.len(r);
+    const uint64_t x = in[i] | (i + 1 < n ? (uint64_t)in[i + 1] << 32 : 0);
+    return x >> (at & 31) & (((uint64_t)1 << b) - 1);
+  };
+  bool undecided = false;
+  auto carryInto = [&](uint32_t k) -> uint32_t {  // of the balanced digits below
+    for (int m = 0; m < LOOK; ++m) {
+      if (k == 0) { return 0; }
+      uint32_t b;
+      const uint64_t x = raw(--k, b), half = (uint64_t)1 << (b - 1);
+      if (x != half - 1) { return x >= half; }
+    }
+    undecided = true;
+    return 0;
+  };
+  int d[2];
+  uint32_t carry = carryInto(2 * j);
+  for (int i = 0; i < 2; ++i) {
+    uint32_t b;
+    const uint64_t x = raw(2 * j + i, b) + carry, half = (uint64_t)1 << (b - 1);
+    carry = x >= half;
+    d[i] = (int)((int64_t)x - (carry ? (int64_t)(2 * half) : 0));
+  }
+  if (j == 0) { d[0] += (int)((in[n - 1] >> (J.E & 31)) + carryInto(N)); }  // what is left above bit E
+  *(int2*)((int32_t*)J.words[wi] + digitAt(J, 2 * j)) = make_int2(d[0], d[1]);
+  if (undecided) { atomicOr(&head->undecided, 1u); }
+}
+
 // small[0..31] = the top 32 words (k = N-32 .. N-1), small[32..63] = the bottom 32 words.
 __global__ __launch_bounds__(64) void k_residue(const JobDesc* __restrict__ jobs, int wi) {
   const JobDesc& J = jobs[blockIdx.y];
@@ -564,6 +682,8 @@ extern "C" const OwlKernelEntry owl_kernel_table[] = {
     {"isEqual", (const void*)&k_is_equal, 256},
     {"sum64", (const void*)&k_sum64, 256},
     {"fill32", (const void*)&k_fill32, 256},
+    {"pack", (const void*)&k_pack, 256},
+    {"unpack", (const void*)&k_unpack, 256},
     {"midBase", (const void*)&k_mid_base, 256},
     {"copyWords", (const void*)&k_copy_words, 256},
     {nullptr, nullptr, 0},
