@@ -275,35 +275,7 @@ Gpu::Gpu(u32 E, const FFTConfig& fftIn, const GpuOptions& optIn) : E{E}, fft{fft
   if (rowFixed) {
     // Per row-pass thread and block: which of its words are big and which weight exponents wrap
     // (the tests of wordWeight, src/Gpu.cpp:40-127's bitsCF), so the pass does not recompute them.
-    const u32 T = rowT, F0 = W / T;
-    // thread tid's columns are colBase(tid) + k*T (RowPass::colBase, kfixed.h; tid + k*T in k_rowm)
-    auto colBase = [F0, this](u32 tid) -> u32 {
-      if (rowM) { return tid; }
-      const u32 b = tid & 15, hi = tid & ~15u;
-      if (F0 == 2) { return hi | (b & 3) | ((b >> 3) << 2) | (((b >> 2) & 1) << 3); }
-      if (F0 == 4) { return hi | (b & 1) | (((b >> 3) & 1) << 1) | (((b >> 1) & 3) << 2); }
-      if (F0 == 8) { return hi | ((b >> 3) & 1) | ((b & 7) << 1); }
-      return tid;
-    };
-    std::vector<u64> meta(size_t(nb) * T, 0);
-    for (u32 lb = 0; lb < nb; ++lb) {
-      for (u32 tid = 0; tid < T; ++tid) {
-        u64 m = 0;
-        for (u32 k = 0; k < F0; ++k) {
-          for (u32 r = 0; r < R; ++r) {
-            for (u32 rep = 0; rep < 2; ++rep) {
-              const u32 w = (k * R + r) * 2 + rep;
-              const u32 t = lineW[lb * R + r].e[rep] + colW[colBase(tid) + k * T].e;
-              const bool wrap = t >= N;
-              const bool big = (wrap ? t - N : t) < J.rE;
-              m |= (u64(big) << w) | (u64(wrap) << (32 + w));
-            }
-          }
-        }
-        meta[size_t(lb) * T + tid] = m;
-      }
-    }
-    J.rowMeta = upload(meta);
+    J.rowMeta = alloc<uint64_t>(size_t(nb) * rowT);
   }
   for (int i = 0; i < 3; ++i) { J.freq[i] = alloc<double2>(ND); }
   for (int i = 0; i < 4; ++i) { J.words[i] = alloc<int2>(ND); }
@@ -324,6 +296,11 @@ Gpu::Gpu(u32 E, const FFTConfig& fftIn, const GpuOptions& optIn) : E{E}, fft{fft
   for (int i = 0; i < 4; ++i) { owlCheck(owl_hip_fill32(queue_, J.words[i], 0, 2 * ND), "fill"); }
   jobs_ = Buffer<JobDesc>(1);
   jobs_.write(queue_, {J});
+  if (rowFixed) {
+    const JobDesc* j = jobs_.get();
+    u32 T = rowT, tidColumns = rowM;
+    Kernel("rowMeta")(queue_, (nb * rowT + 255) / 256, 1, 256, 0, {&j, &T, &tidColumns});
+  }
 
   kRow = Kernel(rowKernel);
   if (rowM) {

@@ -9,19 +9,19 @@ static std::pair<long double, long double> rootL(u32 n, u64 k) {
   u32 o = u32(K / n);
   u64 rem = K % n;
   const long double q = 0.785398163397448309615660845819875721L;  // pi/4
-  long double x = q * (long double)rem / (long double)n;
-  long double y = q * (long double)(n - rem) / (long double)n;
-  long double cx = cosl(x), sx = sinl(x), cy = cosl(y), sy = sinl(y);
+  // even octants by x, odd ones by y
+  const long double angle = q * (long double)(o & 1 ? n - rem : rem) / (long double)n;
+  const long double ca = cosl(angle), sa = sinl(angle);
   long double c = 0, s = 0;
   switch (o) {
-    case 0: c = cx; s = sx; break;
-    case 1: c = sy; s = cy; break;
-    case 2: c = -sx; s = cx; break;
-    case 3: c = -cy; s = sy; break;
-    case 4: c = -cx; s = -sx; break;
-    case 5: c = -sy; s = -cy; break;
-    case 6: c = sx; s = -cx; break;
-    default: c = cy; s = -sy; break;
+    case 0: c = ca; s = sa; break;
+    case 1: c = sa; s = ca; break;
+    case 2: c = -sa; s = ca; break;
+    case 3: c = -ca; s = sa; break;
+    case 4: c = -ca; s = -sa; break;
+    case 5: c = -sa; s = -ca; break;
+    case 6: c = sa; s = -ca; break;
+    default: c = ca; s = -sa; break;
   }
   // exact values at multiples of pi/2
   if (rem == 0 && o % 2 == 0) {
@@ -37,9 +37,10 @@ std::pair<double, double> root1(u32 n, u64 k) {
   return {double(c), double(s)};
 }
 
-std::pair<double, double> root1Low(u32 n, u64 k) {
+RootParts root1Parts(u32 n, u64 k) {
   const auto [c, s] = rootL(n, k);
-  return {double(c - (long double)double(c)), double(s - (long double)double(s))};
+  const double ch = double(c), sh = double(s);
+  return {{ch, sh}, {double(c - (long double)ch), double(s - (long double)sh)}};
 }
 
 std::vector<u32> fftPlan(u32 L) {

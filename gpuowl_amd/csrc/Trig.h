@@ -13,8 +13,11 @@ using u64 = uint64_t;
 
 // exp(-2 pi i k / n) = (cos(2 pi k/n), -sin(2 pi k/n)), k reduced exactly to one octant.
 std::pair<double, double> root1(u32 n, u64 k);
-// What root1's rounding leaves off (to the 64 bits of a long double).
-std::pair<double, double> root1Low(u32 n, u64 k);
+// root1 and what its rounding leaves off (to the 64 bits of a long double).
+struct RootParts {
+  std::pair<double, double> high, low;
+};
+RootParts root1Parts(u32 n, u64 k);
 
 // Mixed-radix plan for an L-point FFT: radices in {2..16}, largest first.
 // Empty if L has a prime factor above 13.

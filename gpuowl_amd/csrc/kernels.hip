@@ -633,6 +633,35 @@ __global__ __launch_bounds__(256) void k_copy_words(const JobDesc* __restrict__ 
   for (uint32_t p = blockIdx.x * 256 + threadIdx.x; p < J.ND; p += gridDim.x * 256) { J.words[dst][p] = J.words[src][p]; }
 }
 
+// Word metadata of the specialized row passes (JobDesc::rowMeta): thread tid of block lb has the columns cb + k*T, k < W/T,
+// of its R lines, cb = tid in k_rowm (tidColumns), else RowPass::colBase(tid); its word w = (k*R + r)*2 + rep sets bit w if it
+// is big, bit 32 + w if its weight exponent wraps.
+__global__ __launch_bounds__(256) void k_row_meta(const JobDesc* __restrict__ jobs, uint32_t T, uint32_t tidColumns) {
+  const JobDesc& J = jobs[0];
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= J.nb * T) { return; }
+  const uint32_t lb = i / T, tid = i % T, F0 = J.W / T, b = tid & 15, hi = tid & ~15u;
+  uint32_t cb = tid;
+  if (!tidColumns) {
+    cb = F0 == 2   ? hi | (b & 3) | ((b >> 3) << 2) | (((b >> 2) & 1) << 3)
+         : F0 == 4 ? hi | (b & 1) | (((b >> 3) & 1) << 1) | (((b >> 1) & 3) << 2)
+         : F0 == 8 ? hi | ((b >> 3) & 1) | ((b & 7) << 1)
+                   : tid;
+  }
+  uint64_t m = 0;
+  for (uint32_t k = 0; k < F0; ++k) {
+    const uint32_t ec = J.colW[cb + k * T].e;
+    for (uint32_t r = 0; r < J.R; ++r) {
+      for (uint32_t rep = 0; rep < 2; ++rep) {
+        const uint32_t w = (k * J.R + r) * 2 + rep, t = J.lineW[lb * J.R + r].e[rep] + ec;
+        const bool wrap = t >= J.N;
+        m |= (uint64_t)((wrap ? t - J.N : t) < J.rE) << w | (uint64_t)wrap << (32 + w);
+      }
+    }
+  }
+  ((uint64_t*)J.rowMeta)[i] = m;
+}
+
 // Mid twiddles of the mirrored column pass: out[a*NB0 + j] = exp(-2 pi i a*j / ND), the product of the row's low factor
 // j mod 64 and high factor j div 64 (in: per row a the 64 + nHi factors, each followed by its low part) to about
 // 2^-64, rounded once.
@@ -682,6 +711,7 @@ extern "C" const OwlKernelEntry owl_kernel_table[] = {
     {"isEqual", (const void*)&k_is_equal, 256},
     {"sum64", (const void*)&k_sum64, 256},
     {"fill32", (const void*)&k_fill32, 256},
+    {"rowMeta", (const void*)&k_row_meta, 256},
     {"pack", (const void*)&k_pack, 256},
     {"unpack", (const void*)&k_unpack, 256},
     {"midBase", (const void*)&k_mid_base, 256},
