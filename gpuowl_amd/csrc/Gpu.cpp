@@ -576,18 +576,17 @@ void Gpu::writeDigits(Buf b, const std::vector<int>& digits) {
   finish();
 }
 
-// Device memory for a residue's words behind a PackHead: kept by a job that runs alone, `own` for one of many (which
-// would each hold 2.5 bytes per digit for the rare read or write).
-u32* Gpu::packed(Buffer<u32>& own) {
-  Buffer<u32>& p = keepPacked_ ? packed_ : own;
-  if (!p.get()) { p = Buffer<u32>(sizeof(PackHead) / 4 + nWords(E)); }
-  return p.get();
+// Device memory for a residue's words behind a PackHead: a buffer that a job running alone keeps; for one of many its own
+// second spectrum (8 bytes per digit), which holds something within modMul only.
+u32* Gpu::packed() {
+  if (!keepPacked_) { return reinterpret_cast<u32*>(job_.freq[2]); }
+  if (!packed_.get()) { packed_ = Buffer<u32>(sizeof(PackHead) / 4 + nWords(E)); }
+  return packed_.get();
 }
 
 void Gpu::writeIn(Buf b, const u32* words, size_t n) {
   if (n == nWords(E)) {
-    Buffer<u32> own;
-    u32* dev = packed(own);
+    u32* dev = packed();
     u32* data = dev + sizeof(PackHead) / 4;
     const JobDesc* j = jobs_.get();
     int wi = b;
@@ -638,8 +637,7 @@ void Gpu::readDigitsVia(Buf b, int32_t* staging, int32_t* out) {
 }
 
 bool Gpu::readWords(Buf b, u32* out) {
-  Buffer<u32> own;
-  u32* dev = packed(own);
+  u32* dev = packed();
   u32* data = dev + sizeof(PackHead) / 4;
   const u32 n = nWords(E);
   const JobDesc* j = jobs_.get();

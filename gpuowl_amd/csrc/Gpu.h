@@ -245,7 +245,7 @@ private:
   template<typename T> T* alloc(size_t n);
   template<typename T> T* upload(const std::vector<T>& v);
   void readDigitsVia(Buf b, int32_t* staging, int32_t* out);
-  u32* packed(Buffer<u32>& own);
+  u32* packed();
 };
 
 // Mersenne-prime type-1 PRP residue is 9 (src/Gpu.cpp:1036-1040).
