@@ -174,8 +174,8 @@ def pmc_pass(counter, steps=20, warmup=5):
     return rows
 
 
-def pmc_traffic(kernel_prefix, copy_bytes):
-    """HBM bytes per launch of the kernel whose name starts with kernel_prefix (its most
+def pmc_traffic(kernel_names, copy_bytes):
+    """HBM bytes per launch of the kernel with one of the names (a tuple; its most
     frequent grid), from FETCH_SIZE and WRITE_SIZE, each scaled by what the counter reads
     for the state copy of copy_bytes read + copy_bytes written in the same run."""
     got = {}
@@ -184,7 +184,7 @@ def pmc_traffic(kernel_prefix, copy_bytes):
         if not rows:
             return None
         copy = [v for (k, g), vs in rows.items() if "copyBuffer" in k for v in vs if v * 1024 > copy_bytes / 4]
-        mine = {(k, g): vs for (k, g), vs in rows.items() if k.split("(")[0].split("<")[0].endswith(kernel_prefix)}
+        mine = {(k, g): vs for (k, g), vs in rows.items() if k.split("(")[0].split("<")[0].endswith(kernel_names)}
         if not copy or not mine:
             return None
         key = max(mine, key=lambda kg: len(mine[kg]))
@@ -329,9 +329,9 @@ def main():
     copy_bytes = 8 * N  # the state copy reads 8*N bytes and writes 8*N bytes
     traffic = None
     if not a.no_pmc:
-        prefix = "k_rowx" if names[dom].startswith("rowx") else "k_colx" if names[dom].startswith("colx") else \
-            "k_row" if dom == "row" else "k_col"
-        traffic = pmc_traffic(prefix, copy_bytes)
+        kernel = ("k_rowx", "k_rowm") if names[dom].startswith("rowx") else ("k_colx",) if names[dom].startswith("colx") \
+            else ("k_row",) if dom == "row" else ("k_col",)
+        traffic = pmc_traffic(kernel, copy_bytes)
         note(f"counter passes done: {traffic['bytes'] if traffic else None} HBM bytes per launch")
     roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(achieved / HBM_PEAK_GBS, 4),
