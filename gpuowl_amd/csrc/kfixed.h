@@ -6,6 +6,8 @@
 // loop unrolled) and fewer LDS round trips:
 //   k_colx: a butterfly of each of the pair's columns in registers from the load to the
 //           store, four LDS exchanges (forward plan [C0,C1,C2], inverse [C2,C1,C0]).
+//   k_rowm: as k_rowx, and the first inverse and last forward stages load and store the block directly, 16
+//           elements per thread (1024 x 4 lines, 512 x 4, 256 x 8).
 //   k_rowx: the last inverse stage leaves each thread holding whole columns
 //           (T = W/F0 threads, columns tid + k*T for all R lines), so rounding,
 //           the carry chain, the stairway hand-off and the weighting all run in
@@ -296,8 +298,8 @@ __device__ __forceinline__ void fillColTw(const JobDesc& J, T2* tab, int a0, int
 // that consecutive butterflies write distinct slots; the two columns' regions use different halves of the banks
 // and alternate by 16 lanes.
 // NT: non-temporal loads and stores.
-// Measured (HIP events, us per launch, the pass before it in parentheses): 1024 x 3840 split 38.4 (46.1), 1024 x 2560
-// split 29.4 (35.4), 1024 x 1536 19.1 (23.4), 256 x 2304 18.7 (20.3), 256 x 512 9.2 (13.5).
+// Measured (HIP events, us per launch, the pass before it in parentheses): 1024 x 3840 split 38.6 (46.1), 1024 x 2560
+// split 28.9 (35.4), 1024 x 1536 20.2 (23.4), 256 x 2304 18.9 (20.3), 256 x 512 9.4 (13.5).
 // Values derived from i before and after are computed anew instead of being held in registers.
 #define FRESH(i) asm volatile("" : "+v"(i))
 // Fixes the place of the values in the instruction stream.
@@ -1200,8 +1202,9 @@ __global__ __launch_bounds__(W / F0) void k_rowx(const JobDesc* __restrict__ job
 // LDS positions are sums without bank conflicts on the writes: exchanges 1 and 3 (Ns = 1) pad one slot per 16,
 // exchange 4's blocks are F0 slots further apart; the line strides differ so that lanes of R lines at one
 // position do not meet.
-// Measured (HIP events, us per fused launch, k_rowx in parentheses): 1024 x 3840 split 38.5 (43.4), 1024 x 1536 complex
-// 22.5 (24.2), 64 jobs of 256 x 2304 split 277 (340).
+// Measured (HIP events, us per fused launch, k_rowx in parentheses): 1024 x 3840 split 38.0 (43.4), 1024 x 1536 complex
+// 23.2 (24.2), 64 jobs of 256 x 2304 split 277 (340). Two-line blocks stay with k_rowx, which has more waves for them:
+// 512 x 1152 15.7 (18.1 with 16 elements per thread), 1024 x 1408 20.8 (22.7).
 template<int W, int R, int F0, int F1, bool SPLIT> struct RowM {
   static constexpr int T = W / F0, J = W / 16, F2 = 16, MB = 16 / F1, NB1 = W / F1;
   static_assert(F0 * F1 * F2 == W && R * F0 == 16 && T % 64 == 0 && NB1 % 16 == 0 && J % 16 == 0, "plan");
