@@ -93,10 +93,12 @@ Gpu::Gpu(u32 E, const FFTConfig& fftIn, const GpuOptions& optIn) : E{E}, fft{fft
     opt.colOnePair = tuned.colOnePair;
     tunedLineBlock_ = true;
   }
-  // A job that runs alone takes the split and line block that fill the device, whatever the reference's. In the last 0.3%
-  // below the largest exponent of its FFT it keeps the reference's, whose round-off is smaller by up to 11% (a 512 x 2048
-  // split of 2^21 words against 256 x 4096 in 8-line blocks: mean largest error 0.213 against 0.203 at the limit, and
-  // 0.194 at 0.3% below it).
+  // A job that runs alone takes the split and line block that fill the device, whatever the reference's. Its round-off is up
+  // to 4.2% higher at the same exponent (256:9:256, 512 x 1152 for 256 x 2304; of 36 FFTs whose split or line block
+  // differs, 9 by more than 3%; about 1% of it is k_rowx's twiddles as products of two). So the last 0.3% below an FFT's
+  // limit keep the reference's split: 0.3% fewer bits per word take 7 to 8% off the round-off, and at the rule's edge it
+  // is at least 3.5% below the reference split's at the limit, for every FFT (256:9:256 0.1496 and 0.1551, 256:16:256
+  // 0.1516 and 0.1591).
   const bool alone = !opt.shared && !opt.lineBlock && !opt.generic && !opt.colOneRegion && E <= 0.997 * fft.maxExp();
   if (opt.width) {
     if (ND % opt.width) { throw std::invalid_argument("width does not divide the FFT length"); }
