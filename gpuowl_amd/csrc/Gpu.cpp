@@ -578,28 +578,29 @@ void Gpu::writeDigits(Buf b, const std::vector<int>& digits) {
   finish();
 }
 
-// Device memory for a residue's words behind a PackHead: a buffer that a job running alone keeps; for one of many its own
-// second spectrum (8 bytes per digit), which holds something within modMul only.
-u32* Gpu::packed() {
-  if (!keepPacked_) { return reinterpret_cast<u32*>(job_.freq[2]); }
-  if (!packed_.get()) { packed_ = Buffer<u32>(sizeof(PackHead) / 4 + nWords(E)); }
-  return packed_.get();
+// Device memory for a residue's words behind two PackHeads: a buffer that a job running alone keeps; for one of many its
+// own second spectrum (8 bytes per digit), which holds something within modMul only.
+PackHead* Gpu::packed() {
+  if (!keepPacked_) { return reinterpret_cast<PackHead*>(job_.freq[2]); }
+  if (!packed_.get()) { packed_ = Buffer<u32>(2 * sizeof(PackHead) / 4 + nWords(E)); }
+  return reinterpret_cast<PackHead*>(packed_.get());
 }
 
 void Gpu::writeIn(Buf b, const u32* words, size_t n) {
-  if (n == nWords(E)) {
-    u32* dev = packed();
-    u32* data = dev + sizeof(PackHead) / 4;
-    const JobDesc* j = jobs_.get();
-    int wi = b;
-    PackHead head;
-    owlCheck(owl_hip_fill32(queue_, dev, 0, sizeof(head) / 4), "fill");
+  PackHead* heads = packed();
+  u32* data = reinterpret_cast<u32*>(heads + 2);
+  const JobDesc* j = jobs_.get();
+  int wi = b;
+  const u32 groups = std::min((ND + 255) / 256, 2048u);
+  PackHead h[2] = {};
+  for (int attempt = 0; n == nWords(E) && !packHeadsAgree(h, groups); ++attempt) {
+    if (attempt == 3) { throw GpuError("persistent GPU read errors"); }
+    owlCheck(owl_hip_fill32(queue_, heads, 0, sizeof(h) / 4), "fill");
     owlCheck(owl_hip_write(queue_, data, words, n * 4, 0), "write");
-    kUnpack(queue_, (ND + 255) / 256, 1, 256, 0, {&j, &wi, &dev, &data});
-    owlCheck(owl_hip_read(queue_, &head, dev, sizeof(head), 1), "read");
-    if (!head.undecided) { return; }
+    kUnpack(queue_, groups, 1, 256, 0, {&j, &wi, &heads, &data});
+    owlCheck(owl_hip_read(queue_, h, heads, sizeof(h), 1), "read");
   }
-  writeDigits(b, expandBits(Words(words, words + n), N, E));
+  if (!h[0].groups || h[0].flags & PACK_UNDECIDED) { writeDigits(b, expandBits(Words(words, words + n), N, E)); }
 }
 
 std::vector<int> Gpu::readDigits(Buf b) {
@@ -639,27 +640,31 @@ void Gpu::readDigitsVia(Buf b, int32_t* staging, int32_t* out) {
 }
 
 bool Gpu::readWords(Buf b, u32* out) {
-  u32* dev = packed();
-  u32* data = dev + sizeof(PackHead) / 4;
+  PackHead* heads = packed();
+  u32* data = reinterpret_cast<u32*>(heads + 2);
   const u32 n = nWords(E);
   const JobDesc* j = jobs_.get();
   int wi = b;
+  u32 packers = std::min((n + 255) / 256, 1024u);
+  const u32 groups = packers + std::min((ND + 255) / 256, 1024u);  // the others sum the digits
   for (int attempt = 0; attempt < 3; ++attempt) {
-    PackHead head;
-    owlCheck(owl_hip_fill32(queue_, dev, 0, sizeof(head) / 4), "fill");
-    kPack(queue_, std::min((n + 255) / 256, 1024u), 1, 256, 0, {&j, &wi, &dev, &data});
-    owlCheck(owl_hip_read(queue_, &head, dev, sizeof(head), 1), "read");
-    if (head.timedOut) { throw GpuError("carry hand-off timed out"); }
-    if (!head.nonZero) { return false; }
-    if (head.undecided) {
-      const Words w = compactBits(readDigits(b), E);
-      std::copy(w.begin(), w.end(), out);
-      return true;
+    PackHead h[2];
+    owlCheck(owl_hip_fill32(queue_, heads, 0, sizeof(h) / 4), "fill");
+    kPack(queue_, groups, 1, 256, 0, {&j, &wi, &heads, &data, &packers});
+    owlCheck(owl_hip_read(queue_, h, heads, sizeof(h), 1), "read");
+    switch (packVerdict(h, groups)) {
+      case PackRead::Again: continue;
+      case PackRead::TimedOut: throw GpuError("carry hand-off timed out");
+      case PackRead::Zero: return false;
+      case PackRead::Host: {
+        const Words w = compactBits(readDigits(b), E);
+        std::copy(w.begin(), w.end(), out);
+        return true;
+      }
+      case PackRead::Words: break;
     }
     owlCheck(owl_hip_read(queue_, out, data, size_t(n) * 4, 1), "read");
-    u64 sum = 0;
-    for (u32 i = 0; i < n; ++i) { sum += out[i]; }
-    if (sum == head.sum) { return true; }
+    if (packedWordsMatch(out, n, h[0], E)) { return true; }
   }
   throw GpuError("persistent GPU read errors");
 }

@@ -12,6 +12,7 @@
 #include <hip/hip_vector_types.h>
 
 #include "job.h"
+#include "pack.h"
 #include "TrigBufCache.h"
 
 #include <initializer_list>
@@ -239,13 +240,13 @@ private:
   u32 cus_ = 1;         // compute units
   Kernel kRowF[2][2], kColSq[2][2];  // [split][streamed]: fused row pass (rowM), squaring column pass (colX_)
   Kernel kRow, kCol, kCarryB, kCarryFix, kWordsIn, kWordsOut, kResidue, kIsEqual, kSum64, kCopy, kPack, kUnpack;
-  Buffer<u32> packed_;       // PackHead and a residue's words, kept by a job that runs alone
+  Buffer<u32> packed_;       // two PackHeads and a residue's words, kept by a job that runs alone
   bool keepPacked_ = false;
 
   template<typename T> T* alloc(size_t n);
   template<typename T> T* upload(const std::vector<T>& v);
   void readDigitsVia(Buf b, int32_t* staging, int32_t* out);
-  u32* packed();
+  PackHead* packed();
 };
 
 // Mersenne-prime type-1 PRP residue is 9 (src/Gpu.cpp:1036-1040).

@@ -44,15 +44,6 @@ struct ColW {
   uint32_t pad;
 };
 
-// Result of packing or unpacking a residue (k_pack, k_unpack).
-struct PackHead {
-  uint64_t sum;        // of the packed words
-  uint32_t nonZero;    // a digit is not zero
-  uint32_t undecided;  // a carry or a digit is the host's to decide
-  uint32_t timedOut;   // JobDesc::flags[2]
-  uint32_t pad[3];
-};
-
 struct JobDesc {
   uint32_t E, N, ND, W, H, R, nb;   // nb = H / R line blocks
   uint32_t bitsLo;                  // E / N

@@ -16,6 +16,7 @@
 // (readResidue, src/cl/etc.cl:9-15), k_is_equal (isEqual, src/cl/etc.cl:34-41),
 // k_sum64 (sum64, src/cl/etc.cl:19-29).
 #include "kcommon.h"
+#include "pack.h"
 
 // ---------------------------------------------------------------- LDS Stockham FFT
 // Elements per thread staged in registers during one stage. The host only
@@ -475,14 +476,14 @@ __global__ __launch_bounds__(256) void k_words_out(const JobDesc* __restrict__ j
 
 // ---------------------------------------------------------------- residue words <-> digits
 // A residue's E bits in 32-bit words, low first, from and to the balanced digits of a words buffer (the order of
-// k_words_in). head[] (PackHead, zeroed before): what the host needs to know about the result. One thread per word
+// k_words_in). head[2] (zeroed before): what the host needs to know about the result, twice (pack.h). One thread per word
 // or pair of digits; a borrow or carry comes from the nearest lower digit that decides it, nearly always the first one
 // looked at. After LOOK digits that do not (a short residue's zeros), or for a digit that no normalized state
-// holds, the kernel sets `undecided` and the host converts the digits itself.
-// Bound by the copy over the host link: at 139M bits 17 MB, and 31 MB of digits in device memory, whose R-line pieces
-// of 8R bytes a thread's neighbours W*R apart complete in the caches. The host took 31 MB each way and a serial loop
-// over the digits; a residue of 139M bits written and read back 37.5 -> 2.6 ms, at 9.5M bits one power step with three
-// residues moved 6.2 -> 3.2 ms.
+// holds, the kernel sets PACK_UNDECIDED and the host converts the digits itself.
+// Bound by the copies from and to the caller's pageable memory: 17 MB each way at 139M bits in 2.6 ms; the kernels read
+// 31 MB of digits in pieces of 8R bytes that a thread's neighbours W*R apart complete in the caches. The host took
+// 31 MB each way and a serial loop over the digits; a residue of 139M bits written and read back 37.5 -> 2.6 ms, at
+// 9.5M bits one power step with three residues moved 6.2 -> 3.2 ms.
 constexpr int LOOK = 16;
 
 struct Digits {  // positions and lengths of an exponent's digits
@@ -503,14 +504,55 @@ __device__ __forceinline__ size_t digitAt(const JobDesc& J, uint32_t k) {
   return 2 * ((size_t)(l / J.R) * J.W * J.R + (size_t)c * J.R + l % J.R) + (k & 1);
 }
 
-__global__ __launch_bounds__(256) void k_pack(const JobDesc* __restrict__ jobs, int wi, PackHead* head, uint32_t* out) {
+// A group's share of both heads.
+__device__ __forceinline__ void reportPack(PackHead* head, uint64_t sum, uint64_t digits, uint32_t flags) {
+  __shared__ uint64_t sums[4], values[4];
+  __shared__ uint32_t bits[4];
+  for (int off = 32; off > 0; off >>= 1) {
+    sum += __shfl_xor(sum, off, 64);
+    digits += __shfl_xor(digits, off, 64);
+    flags |= __shfl_xor(flags, off, 64);
+  }
+  const int wave = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) == 0) { sums[wave] = sum, values[wave] = digits, bits[wave] = flags; }
+  __syncthreads();
+  if (threadIdx.x < 2) {
+    PackHead& h = head[threadIdx.x];
+    sum = sums[0] + sums[1] + sums[2] + sums[3];
+    digits = values[0] + values[1] + values[2] + values[3];
+    flags = bits[0] | bits[1] | bits[2] | bits[3];
+    if (sum) { atomicAdd((unsigned long long*)&h.sum, (unsigned long long)sum); }
+    if (digits) { atomicAdd((unsigned long long*)&h.digits, (unsigned long long)digits); }
+    if (flags) { atomicOr(&h.flags, flags); }
+    atomicAdd(&h.groups, 1u);
+  }
+}
+
+// The first `packers` groups pack; the others read the digits again, in memory order, and sum what they are worth mod
+// 2^32 - 1, so that a digit misread on either side shows (one launch: the two run side by side).
+__global__ __launch_bounds__(256) void k_pack(const JobDesc* __restrict__ jobs, int wi, PackHead* head, uint32_t* out,
+                                              uint32_t packers) {
   const JobDesc& J = jobs[0];
   const int32_t* w = (const int32_t*)J.words[wi];
   const Digits D(J);
   const uint32_t n = (J.E - 1) / 32 + 1, N = J.N;
-  uint64_t sum = 0;
-  bool undecided = false, nonZero = false;
-  for (uint32_t p = blockIdx.x * 256 + threadIdx.x; p < n; p += gridDim.x * 256) {
+  uint64_t sum = 0, digits = 0;
+  bool undecided = false, nonZero = false, negative = false;
+  if (blockIdx.x >= packers) {
+    int64_t acc = 0;
+    for (uint32_t p = (blockIdx.x - packers) * 256 + threadIdx.x; p < J.ND; p += (gridDim.x - packers) * 256) {
+      const int2 d = J.words[wi][p];
+      const uint32_t r = p % J.R, c = p / J.R % J.W, l = p / J.R / J.W * J.R + r, k = 2 * (l + J.H * c);
+      uint32_t rem = D.rem(k);
+      const uint32_t at = (uint32_t)D.pos(k), next = at + D.len(rem);
+      const int64_t x = (int64_t)((uint64_t)(int64_t)d.x << (at & 31)), y = (int64_t)((uint64_t)(int64_t)d.y << (next & 31));
+      acc += (x >> 32) + (uint32_t)x + (y >> 32) + (uint32_t)y;
+      nonZero |= (d.x | d.y) != 0;
+    }
+    acc %= 0xffffffffll;
+    digits = (uint64_t)(acc < 0 ? acc + 0xffffffffll : acc);
+  }
+  for (uint32_t p = blockIdx.x * 256 + threadIdx.x; blockIdx.x < packers && p < n; p += packers * 256) {
     const uint64_t bit = 32 * (uint64_t)p;
     uint32_t k = (uint32_t)(bit * N / J.E), r = D.rem(k);
     int64_t borrow = 0;
@@ -523,6 +565,7 @@ __global__ __launch_bounds__(256) void k_pack(const JobDesc* __restrict__ jobs, 
       }
       undecided |= d == 0;
       borrow = d < 0 ? -1 : 0;
+      negative |= p == 0 && d < 0;
     }
     uint64_t acc = 0;
     uint32_t have = 0, skip = (uint32_t)(bit - D.pos(k));
@@ -544,21 +587,15 @@ __global__ __launch_bounds__(256) void k_pack(const JobDesc* __restrict__ jobs, 
     out[p] = (uint32_t)acc;
     sum += (uint32_t)acc;
   }
-  for (int off = 32; off > 0; off >>= 1) { sum += __shfl_xor(sum, off, 64); }
-  const bool anyU = __any(undecided), anyN = __any(nonZero);
-  if ((threadIdx.x & 63) == 0) {
-    atomicAdd((unsigned long long*)&head->sum, (unsigned long long)sum);
-    if (anyU) { atomicOr(&head->undecided, 1u); }
-    if (anyN) { atomicOr(&head->nonZero, 1u); }
-  }
-  if (blockIdx.x == 0 && threadIdx.x == 0) { head->timedOut = J.flags[2]; }
+  const bool late = blockIdx.x == 0 && threadIdx.x == 0 && J.flags[2];
+  reportPack(head, sum, digits, (nonZero ? PACK_NONZERO : 0) | (undecided ? PACK_UNDECIDED : 0) |
+                                    (negative ? PACK_NEGATIVE : 0) | (late ? PACK_TIMED_OUT : 0));
 }
 
 __global__ __launch_bounds__(256) void k_unpack(const JobDesc* __restrict__ jobs, int wi, PackHead* head, const uint32_t* in) {
   const JobDesc& J = jobs[0];
   const Digits D(J);
-  const uint32_t n = (J.E - 1) / 32 + 1, N = J.N, j = blockIdx.x * 256 + threadIdx.x;
-  if (j >= J.ND) { return; }
+  const uint32_t n = (J.E - 1) / 32 + 1, N = J.N;
   auto raw = [&](uint32_t k, uint32_t& b) -> uint64_t {
     uint32_t r = D.rem(k);
     const uint64_t at = D.pos(k);
@@ -578,17 +615,19 @@ __global__ __launch_bounds__(256) void k_unpack(const JobDesc* __restrict__ jobs
     undecided = true;
     return 0;
   };
-  int d[2];
-  uint32_t carry = carryInto(2 * j);
-  for (int i = 0; i < 2; ++i) {
-    uint32_t b;
-    const uint64_t x = raw(2 * j + i, b) + carry, half = (uint64_t)1 << (b - 1);
-    carry = x >= half;
-    d[i] = (int)((int64_t)x - (carry ? (int64_t)(2 * half) : 0));
+  for (uint32_t j = blockIdx.x * 256 + threadIdx.x; j < J.ND; j += gridDim.x * 256) {
+    int d[2];
+    uint32_t carry = carryInto(2 * j);
+    for (int i = 0; i < 2; ++i) {
+      uint32_t b;
+      const uint64_t x = raw(2 * j + i, b) + carry, half = (uint64_t)1 << (b - 1);
+      carry = x >= half;
+      d[i] = (int)((int64_t)x - (carry ? (int64_t)(2 * half) : 0));
+    }
+    if (j == 0) { d[0] += (int)((in[n - 1] >> (J.E & 31)) + carryInto(N)); }  // what is left above bit E
+    *(int2*)((int32_t*)J.words[wi] + digitAt(J, 2 * j)) = make_int2(d[0], d[1]);
   }
-  if (j == 0) { d[0] += (int)((in[n - 1] >> (J.E & 31)) + carryInto(N)); }  // what is left above bit E
-  *(int2*)((int32_t*)J.words[wi] + digitAt(J, 2 * j)) = make_int2(d[0], d[1]);
-  if (undecided) { atomicOr(&head->undecided, 1u); }
+  reportPack(head, 0, 0, undecided ? PACK_UNDECIDED : 0);
 }
 
 // small[0..31] = the top 32 words (k = N-32 .. N-1), small[32..63] = the bottom 32 words.
