@@ -324,6 +324,7 @@ def main():
     alg = {"row": 16 * N, "col": 16 * N}
     kernels = {"col": us_col, "row": us_row}
     names = {"row": g.row_kernel, "col": g.col_kernel}
+    launched = dict(zip(("row", "col"), g.launched()))
     dom = max(kernels, key=kernels.get)
     achieved = alg[dom] / (kernels[dom] * 1e-6) / 1e9
     copy_bytes = 8 * N  # the state copy reads 8*N bytes and writes 8*N bytes
@@ -336,7 +337,7 @@ def main():
     roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(achieved / HBM_PEAK_GBS, 4),
                 "traffic": traffic["bytes"] if traffic else None,
-                "kernel": f"{names[dom]} ({'row pass: fused carry' if dom == 'row' else 'column pass: middle + square'})",
+                "kernel": f"{launched[dom]} ({'row pass: fused carry' if dom == 'row' else 'column pass: middle + square'})",
                 "alg_bytes_per_launch": alg[dom],
                 "us_per_launch": {"col": round(us_col, 2), "row": round(us_row, 2)},
                 "traffic_detail": traffic,

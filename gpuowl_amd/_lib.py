@@ -96,6 +96,7 @@ SIGNATURES = {
     "owl_gpu_create": [u32, cp, i32, u32, P(vp)],
     "owl_gpu_destroy": [vp],
     "owl_gpu_info": [vp, P(GpuInfo)],
+    "owl_gpu_launched": [vp, u32, cp, C.c_size_t, cp, C.c_size_t],
     "owl_gpu_write_words": [vp, i32, P(u32), u32],
     "owl_gpu_read_words": [vp, i32, P(u32), u32, P(i32)],
     "owl_gpu_write_digits": [vp, i32, P(i32), u32],
@@ -142,6 +143,7 @@ SIGNATURES = {
     "owl_batch_destroy": [vp],
     "owl_batch_info": [vp, P(u32), P(u32), P(u64)],
     "owl_batch_job_info": [vp, u32, P(GpuInfo)],
+    "owl_batch_launched": [vp, u32, cp, C.c_size_t, cp, C.c_size_t],
     "owl_batch_prp": [vp, u32, u32, u32, P(u64), u32, u32, P(PrpResult)],
     "owl_batch_arm_fault": [vp, u32, u32],
     "owl_batch_ll": [vp, u32, P(u64), u32, u32, P(LLResult)],

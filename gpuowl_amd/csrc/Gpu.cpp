@@ -435,9 +435,7 @@ void Gpu::rowFused(bool ll, u32 roeSlot, Launch L) {
   int mode = ROW_FUSED, fi = 0, wi = 0, opts = (ll ? 1 : 0) | (rowChunked ? 4 : 0);
   u32 tag = nextStairTag();
   const u32 groups = rowChunked ? 8 * ((nb + 7) / 8 + 1) : nb + 1;
-  const bool split = rowM && rowSplit(L.n);
-  const Kernel& k = rowM ? kRowF[split][streamed(L.n)] : kRow;
-  k(L.q, groups, L.n, rowT, split ? rowLdsS : rowLds, {&L.jobs, &mode, &fi, &wi, &opts, &roeSlot, &tag});
+  rowSquaring(L.n)(L.q, groups, L.n, rowT, rowM && rowSplit(L.n) ? rowLdsS : rowLds, {&L.jobs, &mode, &fi, &wi, &opts, &roeSlot, &tag});
 }
 
 void Gpu::rowLeadInTo(Buf in, int freqIdx, Launch L) {
@@ -480,10 +478,13 @@ bool Gpu::colSplit(u32 nJobs) const { return haveSplit && u64(W / 2) * nJobs >= 
 
 std::string Gpu::colKernelFor(u32 nJobs) const { return colSplit(nJobs) ? colOne_ + "m" : colOne_; }
 
+const Kernel& Gpu::rowSquaring(u32 nJobs) const { return rowM ? kRowF[rowSplit(nJobs)][streamed(nJobs)] : kRow; }
+const Kernel& Gpu::colSquaring(u32 nJobs) const { return colX_ ? kColSq[colSplit(nJobs)][streamed(nJobs)] : kCol; }
+
 void Gpu::colPass(int mode, int fi, int oi, Launch L) {
-  const bool split = mode == COL_SQUARE && colSplit(L.n);
-  const Kernel& k = colX_ && mode == COL_SQUARE ? kColSq[split][streamed(L.n)] : kCol;
-  k(L.q, W / 2, L.n, colT, split ? colSplitLds : colLds, {&L.jobs, &mode, &fi, &oi});
+  const bool squaring = mode == COL_SQUARE;
+  const Kernel& k = squaring ? colSquaring(L.n) : kCol;
+  k(L.q, W / 2, L.n, colT, squaring && colSplit(L.n) ? colSplitLds : colLds, {&L.jobs, &mode, &fi, &oi});
 }
 
 void Gpu::colSquare(Launch L) { colPass(COL_SQUARE, 0, 0, L); }

@@ -84,7 +84,7 @@ public:
   const FFTConfig fft;
   int device = 0;  // the HIP device the engine's queue and buffers are on
   u32 N, ND, W, H, R, nb, rowT, colT, rowLds, colLds;
-  std::string rowKernel, colKernel;  // colKernel: what a launch of this job alone runs
+  std::string rowKernel, colKernel;  // the passes, whose variants (below) share their names but for colx's "m"
   bool rowChunked = false;           // fused row launches in chunked per-XCD block order (nb >= 8)
   // Variants of the squaring's passes, chosen per launch by its number of jobs: exchanges of real and imaginary
   // parts one after the other (split) or of complex elements, plain or non-temporal (streamed) accesses.
@@ -93,7 +93,10 @@ public:
   bool rowSplit(u32 nJobs) const;
   bool colSplit(u32 nJobs) const;
   bool streamed(u32 nJobs) const;
-  std::string colKernelFor(u32 nJobs) const;  // the column kernel a launch of nJobs jobs runs
+  std::string colKernelFor(u32 nJobs) const;  // colKernel for a launch of nJobs jobs ("m": split)
+  // what a fused squaring of nJobs jobs launches
+  const Kernel& rowSquaring(u32 nJobs) const;
+  const Kernel& colSquaring(u32 nJobs) const;
   bool useLongCarry;
   std::vector<u32> rowPlan, colPlan;
 

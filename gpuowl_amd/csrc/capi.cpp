@@ -162,6 +162,14 @@ void fillInfo(const Gpu& G, owl_gpu_info_t* info) {
   }
 }
 
+int owl_gpu_launched(owl_gpu g, uint32_t jobs, char* row, size_t rowLen, char* col, size_t colLen) {
+  return guarded([&] {
+    if (!jobs) { throw std::invalid_argument("no jobs"); }
+    snprintf(row, rowLen, "%s", g->gpu->rowSquaring(jobs).name().c_str());
+    snprintf(col, colLen, "%s", g->gpu->colSquaring(jobs).name().c_str());
+  });
+}
+
 int owl_gpu_write_words(owl_gpu g, int b, const uint32_t* words, uint32_t n) {
   return guarded([&] { g->gpu->writeIn(buf(b), words, n); });
 }
@@ -817,6 +825,15 @@ int owl_batch_job_info(owl_batch b, uint32_t job, owl_gpu_info_t* info) {
     // the column kernel of the job's group launches (the split variant in a large group)
     const GpuBatch::Group& g = b->batch->groupOf(job);
     snprintf(info->colKernel, sizeof(info->colKernel), "%s", g.lead->colKernelFor(u32(g.index.size())).c_str());
+  });
+}
+
+int owl_batch_launched(owl_batch b, uint32_t job, char* row, size_t rowLen, char* col, size_t colLen) {
+  return guarded([&] {
+    const GpuBatch::Group& g = b->batch->groupOf(job);
+    const u32 n = u32(g.index.size());
+    snprintf(row, rowLen, "%s", g.lead->rowSquaring(n).name().c_str());
+    snprintf(col, colLen, "%s", g.lead->colSquaring(n).name().c_str());
   });
 }
 

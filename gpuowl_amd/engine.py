@@ -86,6 +86,12 @@ class Gpu:
         except Exception:
             pass
 
+    def launched(self, jobs=1):
+        """(row, column) kernel of a fused squaring of `jobs` jobs of this geometry in one launch."""
+        row, col = C.create_string_buffer(32), C.create_string_buffer(32)
+        check(self.lib.owl_gpu_launched(self.h, jobs, row, 32, col, 32))
+        return row.value.decode(), col.value.decode()
+
     # ---- state I/O
     def write_words(self, buf, words):
         arr = (C.c_uint32 * len(words))(*words)
@@ -282,6 +288,12 @@ class Batch:
         check(self.lib.owl_batch_job_info(self.h, i, C.byref(info)))
         return {"E": info.E, "N": info.N, "spec": info.spec.decode(), "row": info.rowKernel.decode(),
                 "col": info.colKernel.decode(), "R": info.R, "long_carry": bool(info.longCarry)}
+
+    def launched(self, i):
+        """(row, column) kernel of the fused squarings that job i shares."""
+        row, col = C.create_string_buffer(32), C.create_string_buffer(32)
+        check(self.lib.owl_batch_launched(self.h, i, row, 32, col, 32))
+        return row.value.decode(), col.value.decode()
 
     def arm_fault(self, job, k):
         check(self.lib.owl_batch_arm_fault(self.h, job, k))

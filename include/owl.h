@@ -26,7 +26,7 @@ typedef struct {
   uint32_t maxExp;
   int longCarry;
   char spec[64];     /* reference FFT spec, e.g. "1K:15:256:202" */
-  char rowKernel[32], colKernel[32];   /* the row / column pass kernels in use */
+  char rowKernel[32], colKernel[32];   /* the row / column passes (owl_gpu_launched: their variants) */
 } owl_gpu_info_t;
 
 typedef struct {
@@ -73,6 +73,9 @@ enum { OWL_LONG_CARRY = 1, OWL_GENERIC = 2, OWL_COL_ONE_REGION = 4, OWL_COL_ONE_
 int owl_gpu_create(uint32_t E, const char* spec, int flags, uint32_t lineBlock, owl_gpu* gpu);
 int owl_gpu_destroy(owl_gpu gpu);
 int owl_gpu_info(owl_gpu gpu, owl_gpu_info_t* info);
+/* The kernels that a fused squaring of `jobs` jobs of this geometry in one launch runs: the variant of the row and column pass
+ * named in owl_gpu_info_t, which the number of jobs and the size of their states decide. */
+int owl_gpu_launched(owl_gpu gpu, uint32_t jobs, char* row, size_t rowLen, char* col, size_t colLen);
 
 /* Gpu::writeIn / readData (src/Gpu.cpp:801-811, 707-709): packed residue words, (E-1)/32+1 u32.
  * read: *isZero = 1 and no words written when the residue is all zero. */
@@ -253,6 +256,8 @@ int owl_batch_create(const uint32_t* exponents, uint32_t n, const char* spec, in
 int owl_batch_destroy(owl_batch batch);
 int owl_batch_info(owl_batch batch, uint32_t* nJobs, uint32_t* nGroups, uint64_t* totalWords);
 int owl_batch_job_info(owl_batch batch, uint32_t job, owl_gpu_info_t* info);
+/* owl_gpu_launched for the launches that the job shares */
+int owl_batch_launched(owl_batch batch, uint32_t job, char* row, size_t rowLen, char* col, size_t colLen);
 int owl_batch_prp(owl_batch batch, uint32_t iters, uint32_t blockSize, uint32_t checkStep, uint64_t* res,
                   uint32_t resStep, uint32_t resCap, owl_prp_result_t* out);
 int owl_batch_arm_fault(owl_batch batch, uint32_t job, uint32_t k);
