@@ -22,10 +22,11 @@ u32 pow2AtLeast(u32 x, u32 lo, u32 hi) {
 }
 
 // Width of the W x H split of ND points for a job that runs alone, 0 where the rule has none: the smallest of 256, 512
-// and 1024 with a column pass of at most 2048 lines, and 1024 up to its 4096. Fewer columns than 512 leave
-// compute units without a column pair; more lines per column only lengthen every group's chain of stages.
-// Measured, us per squaring (2-line blocks): ND = 589,824: 256 x 2304 30.1, 512 x 1152 27.2; 851,968: 256 x 3328 41.0 (36.6
-// with 8 lines), 512 x 1664 29.9; 458,752: 256 x 1792 25.8; 1,179,648: 512 x 2304 38.7, 1024 x 1152 34.3.
+// and 1024 with a column pass of at most 2048 lines, and 1024 up to its 4096. More lines per column lengthen every group's
+// chain of stages; fewer columns leave compute units without a column pair (256 columns are 128 pairs for 256 units), which
+// weighs less only while columns are short. Measured, us per squaring in two-line blocks, W = 256 / 512 / 1024: ND = 262,144
+// 18.5 / 18.8; 393,216 23.0 / 21.3; 524,288 27.0 / 24.1 / 25.5; 589,824 31.0 / 27.1; 851,968 41.0 / 29.9; 1,179,648
+// (512 x 2304) 38.7 / 34.3. With 256 columns of 1536 and 2048 lines the line at 2048 gives up 7 and 11%.
 u32 aloneWidth(u32 ND) {
   for (u32 w = 256; w <= 1024; w *= 2) {
     const u32 h = ND / w;
@@ -456,11 +457,11 @@ void Gpu::carryAll(Buf b, Launch L) {
   kCarryFix(L.q, 1, L.n, 256, 0, {&L.jobs, &wi, &co});
 }
 
-// Whether a launch of nJobs jobs streams the state with non-temporal accesses: when the states together fit the
-// L2s (which then write back early instead of at the end of the launch) and when they exceed the 256 MB
-// Infinity Cache. Between, and below 6 MB, plain accesses are faster. Measured, us per squaring,
-// non-temporal / plain: 2 MB 16.4 / 15.7, 9.4 MB 31.2 / 33.8, 25 MB 37.0 / 40.1, 42 MB 56.3 / 57.9, 50 MB 64.8 / 65.2,
-// 63 MB 77.0 / 74.2; batches of 200 MB 262 / 235, 604 MB 639 / 692.
+// Whether a launch of nJobs jobs streams the state with non-temporal accesses, in k_colx and k_rowm (k_rowx's are
+// fixed by its width): when the states together take 6 to 56 MB, and beyond the 256 MB Infinity Cache. The first two lines
+// are where the measurements cross, not a cache's size (the L2s hold 32 MB); us per squaring, non-temporal / plain: 2 MB
+// 16.4 / 15.7, 9.4 MB 31.2 / 33.8, 25 MB 37.0 / 40.1, 42 MB 56.3 / 57.9, 50 MB 64.8 / 65.2, 63 MB 77.0 / 74.2; batches
+// of 200 MB 262 / 235, 604 MB 639 / 692.
 bool Gpu::streamed(u32 nJobs) const {
   const u64 bytes = 8ull * N * nJobs;
   return bytes >= (6u << 20) && (bytes <= (56u << 20) || bytes > (256u << 20));

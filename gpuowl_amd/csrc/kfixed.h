@@ -299,7 +299,7 @@ __device__ __forceinline__ void fillColTw(const JobDesc& J, T2* tab, int a0, int
 // and alternate by 16 lanes.
 // NT: non-temporal loads and stores.
 // Measured (HIP events, us per launch, the pass before it in parentheses): 1024 x 3840 split 38.6 (46.1), 1024 x 2560
-// split 28.9 (35.4), 1024 x 1536 20.2 (23.4), 256 x 2304 18.9 (20.3), 256 x 512 9.4 (13.5).
+// split 28.9 (35.4), 1024 x 1536 20.2 (23.4), 256 x 2304 18.9 (20.3), 256 x 512 9.5 (13.5).
 // Values derived from i before and after are computed anew instead of being held in registers.
 #define FRESH(i) asm volatile("" : "+v"(i))
 // Fixes the place of the values in the instruction stream.
@@ -890,15 +890,15 @@ template<int W, int R, int F0, int F1, int F2> struct RowPass {
   static constexpr int NL = LW / T;  // state elements per thread
   static constexpr int REG = rowRegion<W, R>();
   static constexpr bool LDS_TW = W >= 512;
-  // the block streams through with non-temporal accesses from W = 512 up
+  // k_rowx streams the block with non-temporal accesses from W = 512 up
   static constexpr bool NT = W >= 512;
   using Tw = std::conditional_t<LDS_TW, RowTw<W, F1, F2>, GlobalTw>;
 
   // Thread tid owns the columns colBase(tid) + k*T (k < F0): colBase permutes the low four bits of
   // tid so that the first forward stage's LDS writes (positions colBase*F0 + k, one per lane) of
   // 8 consecutive lanes fall in 8 distinct bank slots (LDS writes serve 8 lanes per cycle, 16-byte
-  // slots mod 8); with colBase = tid they pair up for F0 = 2, 4 and 8. The host lays out the word
-  // metadata with the same permutation.
+  // slots mod 8); with colBase = tid they pair up for F0 = 2, 4 and 8. k_row_meta lays out the
+  // word metadata with the same permutation.
   __device__ __forceinline__ static int colBase(int tid) {
     const int b = tid & 15, hi = tid & ~15;
     if constexpr (F0 == 2) {
